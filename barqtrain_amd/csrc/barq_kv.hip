@@ -2047,6 +2047,7 @@ const char* barq_kv_status_string(int status) {
     case BARQ_KV_ERR_INVALID: return "invalid argument (pointer, size, stride or alignment)";
     case BARQ_KV_ERR_LAUNCH: return "HIP kernel launch failed";
     case BARQ_KV_ERR_SCRATCH: return "request exceeds the static scratch (BARQ_KV_SCRATCH_BYTES per GPU)";
+    case BARQ_KV_ERR_UNSUPPORTED: return "no kernel for this form of the request";
     default: return "unknown status";
   }
 }

@@ -84,13 +84,13 @@ __device__ __forceinline__ float e4m3_decode(uint32_t c) {
   return __uint_as_float(__float_as_uint(mag) | sign);
 }
 
-// Smallest e with a <= 448 * 2^e (0 for a == 0), clamped to [-127, 127]: with a = m * 2^x,
-// m in [0.5, 1), e = x - 9, plus 1 when m > 0.875 (448 = 0.875 * 2^9).
+// Smallest e with a <= 448 * 2^e (0 for a == 0), at least -127, for finite a >= 0: 448 = 1.75 * 2^8,
+// so e is a's exponent minus 8, plus 1 when its significand passes 1.75 -- a mantissa above
+// 0x600000, which adding 0x1FFFFF carries into the exponent field.  (A denormal's field of 0 gives
+// less than -127, as its exponent would.)
 __device__ __forceinline__ int group_exponent(float a) {
-  if (a == 0.0f) return 0;
-  int x;
-  const float m = frexpf(a, &x);
-  return max(-127, min(127, x - 9 + (m > 0.875f ? 1 : 0)));
+  const uint32_t u = __float_as_uint(a);
+  return u == 0 ? 0 : max(-127, (int)((u + 0x1FFFFFu) >> 23) - 135);
 }
 
 __device__ __forceinline__ float finite_abs(float v) {

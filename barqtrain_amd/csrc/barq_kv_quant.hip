@@ -98,8 +98,7 @@ struct ColdPtrs {
 };
 
 // ---------------------------------------------------------------------------------------------
-// Compress: workgroup per row.  quantise_page serves any geometry; quantise_regs below (one
-// round trip of loads per page) the common two-byte ones.
+// Compress: workgroup per row, any geometry (quant_blocks_kernel below takes the common ones).
 // ---------------------------------------------------------------------------------------------
 
 struct CompressArgs {
@@ -295,188 +294,449 @@ __global__ void __launch_bounds__(kThreads) compress_kernel(const CompressArgs a
   if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);
 }
 
-// Register-resident compress for 16-byte vectors of 2-byte elements, when a token's G = C / 8
-// vectors divide the workgroup (G | 256), a page holds NV * 256 vectors and D / 8 is a power of
-// two: thread t holds vectors t + 256 i (i < NV) of a page's K and V -- channel group t % G of
-// tokens t / G + i * 256 / G -- so a page costs one round trip of loads, issued (for a row's first
-// block) while the cold pages are popped.  Key maxima over the page's tokens combine the 256 / G
-// threads of a channel group through LDS; value maxima over a (token, head) combine the head's
-// D / 8 adjacent lanes with shuffles.  The codes and scales are quantise_page's: maxima of finite
-// magnitudes, group_exponent, e4m3_encode of x * 2^-e.  A row's blocks take the cold pages its one
-// pop reserves in block order (free_cold[top - 1], [top - 2], ...), and their hot pages go back
-// with one push, in block order.
-constexpr int kRegsMaxChannels = 2048;  // C = G * 8 with G | 256
+// ---------------------------------------------------------------------------------------------
+// Blocks quantised by whole workgroups, a wave to each (K or V, head) of a block: the compress of
+// pools whose pages divide into waves (quant_blocks_vectors below), and an append of any number
+// of tokens that quantises what passes the residual window straight from the input.
+//
+// A unit = one head of a block's K (or V), NV vectors of 16 bytes per lane: lane l holds column
+// l % vd (vd = vectors per head row) of tokens l / vd + i * 64 / vd.  Key maxima over the page's
+// tokens and value maxima over head_dim then cross lanes of one wave only -- no LDS, no barrier --
+// and a block's units are independent, so a workgroup of up to 16 waves takes a block in one round
+// trip of loads.  (One 256-thread workgroup per row, its blocks one after the other through LDS,
+// left 240 of 256 CUs idle on a batch of 16: 33 us for four pages a row.)
+//
+// Tiles (row, i): i < nnew is the i-th block that receives new tokens -- a block the commit has
+// just mapped to a cold page is quantised from the input, one that stays behind the frontier is
+// copied to its hot page, one that was hot before (the row's partial block, blocks a crop
+// re-opened) is quantised from its page and the input; i >= nnew are the row's older hot blocks.
+// Blocks that were hot take their cold page and return their hot page through atomics on the stack
+// tops, which no other part of the launch moves the other way.
+//
+// Bound: HBM (the input read once, codes and scales written once), then the round trips of a
+// workgroup's only block.  A 16 x 1000-token prompt of the 8 x 128 bf16 shape: 24.7 us for 95 MB
+// after a 6.8 us plan, against 16 chunks of an append and a compress each, 9.2 + 33 us.
+// ---------------------------------------------------------------------------------------------
 
+// Tiles per row that look for older hot blocks: a decode step has one such block every page_size
+// steps, an append of 64 tokens four (page size 16).
+constexpr int kOldTiles = 4;
+
+struct QuantArgs {
+  barq_kv_pool p;
+  ColdPtrs c;
+  const char* in[2];      // key, value states (append)
+  int64_t isb, ish, ist;  // input strides, elements
+  int32_t tokens;         // appended tokens, already counted in seq_lens (0: compress only)
+  int32_t ahead;          // compress: tokens the rows are about to receive
+  int32_t nnew;           // tiles per row of blocks that receive tokens
+  int32_t vd_log2;        // vectors per head row
+  FastDiv div_page;
+  FastDiv div_tiles;      // nnew + kOldTiles
+};
+
+// The lane, unknown to the optimiser: a unit's per-vector offsets are computed where they are used
+// and not held across the loop over units (16 registers a vector).
+__device__ __forceinline__ int opaque_lane() {
+  int lane = threadIdx.x & (kWave - 1);
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
+// Loads unit (kv, h) of the block whose positions start at s0: from hot page hp (if any), and
+// positions from len on -- the launch's tokens -- from the input.  Lane offsets fit 32 bits.
 template <int KIND, int NV>
-struct PageRegs {
-  using Raw = typename RawC<16>::T;
-  Raw k[NV], v[NV];
-
-  __device__ void load(const barq_kv_pool& p, int hp, int C) {
-    const Raw* kp = (const Raw*)((const char*)p.key_pages + (int64_t)hp * p.page_size * C * 2);
-    const Raw* vp = (const Raw*)((const char*)p.value_pages + (int64_t)hp * p.page_size * C * 2);
+__device__ __forceinline__ void load_unit(const QuantArgs& a, int b, int kv, int h, int hp, int s0, int len,
+                                          typename RawC<16>::T (&x)[NV]) {
+  using Bits = typename Elem<KIND>::Bits;
+  using V = typename RawC<16>::T;
+  const barq_kv_pool& p = a.p;
+  const int lane = opaque_lane();
+  const int col = (lane & ((1 << a.vd_log2) - 1)) * (16 / (int)sizeof(Bits));
+  const int t0 = lane >> a.vd_log2, step = kWave >> a.vd_log2;
+  const int HD = (int)(p.kv_heads * p.head_dim), P = (int)p.page_size;
+  const Bits* in = (const Bits*)a.in[kv] + ((int64_t)b * a.isb + (int64_t)h * a.ish + (int64_t)(s0 - len) * a.ist);
+  const uint32_t ist = (uint32_t)a.ist;
+  if (hp < 0) {  // uniform: only new tokens
 #pragma unroll
-    for (int i = 0; i < NV; ++i) k[i] = kp[threadIdx.x + kThreads * i];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) v[i] = vp[threadIdx.x + kThreads * i];
+    for (int i = 0; i < NV; ++i)
+      x[i] = __builtin_nontemporal_load((const V*)(in + ((uint32_t)(t0 + i * step) * ist + (uint32_t)col)));
+    return;
   }
-  __device__ static float elem(const Raw& w, int e) {
-    return Elem<KIND>::to_float((uint16_t)(w[e >> 1] >> (16 * (e & 1))));
+  const Bits* page = (const Bits*)(kv ? p.value_pages : p.key_pages) + ((int64_t)hp * P * HD + h * (int)p.head_dim);
+#pragma unroll
+  for (int i = 0; i < NV; ++i) x[i] = __builtin_nontemporal_load((const V*)(page + (uint32_t)((t0 + i * step) * HD + col)));
+  if (s0 + P > len) {  // uniform: the block's last positions are new
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int t = t0 + i * step;
+      const V y = *(const V*)(in + ((uint32_t)max(t, len - s0) * ist + (uint32_t)col));
+      x[i] = s0 + t >= len ? y : x[i];
+    }
+  }
+}
+
+// Magnitudes as bit patterns, whose order is the values': a word holds two of a two-byte type or one
+// fp32.
+template <int KIND>
+struct Mag {
+  static constexpr bool kPacked = KIND != BARQ_KV_FP32;
+  static constexpr uint32_t kMask = kPacked ? 0x7FFF7FFFu : 0x7FFFFFFFu;
+  static constexpr uint32_t kInf = KIND == BARQ_KV_BF16 ? 0x7F80u : KIND == BARQ_KV_FP16 ? 0x7C00u : 0x7F800000u;
+  __device__ static uint32_t max2(uint32_t a, uint32_t b) {
+    if constexpr (kPacked) {
+      using P2 = uint16_t __attribute__((ext_vector_type(2)));
+      return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(P2, a), __builtin_bit_cast(P2, b)));
+    } else {
+      return max(a, b);
+    }
+  }
+  __device__ static bool any_nonfinite(uint32_t m) {
+    if constexpr (kPacked) return (m & 0xFFFFu) >= kInf || (m >> 16) >= kInf;
+    return m >= kInf;
+  }
+  // the word's magnitudes, infinities and NaN as 0
+  __device__ static uint32_t finite(uint32_t w) {
+    const uint32_t m = w & kMask;
+    if constexpr (kPacked) return ((m & 0xFFFFu) >= kInf ? 0u : m & 0xFFFFu) | ((m >> 16) >= kInf ? 0u : m & 0xFFFF0000u);
+    return m >= kInf ? 0u : m;
+  }
+  // element e of word w as a float (e: 0 low, 1 high half)
+  __device__ static float value(uint32_t w, int e) {
+    if constexpr (KIND == BARQ_KV_BF16) return __uint_as_float(e ? w & 0xFFFF0000u : w << 16);
+    if constexpr (KIND == BARQ_KV_FP16) return Elem<KIND>::to_float((uint16_t)(e ? w >> 16 : w));
+    return __uint_as_float(w);
   }
 };
 
+// Codes and scales of unit (kv, h) into cold page cp.  The maxima run on magnitude bits (two
+// elements an operation); the codes are e4m3_encode of x * 2^-e through the hardware conversion
+// (e4m3_encode4's domain), infinities and NaN -- looked for only in units that hold one -- given
+// the NaN code with their sign.
 template <int KIND, int NV>
-__device__ void quantise_regs(const CompressArgs& a, const PageRegs<KIND, NV>& pg, int cp, float* s_red,
-                              int8_t* s_kexp) {
-  using Regs = PageRegs<KIND, NV>;
+__device__ __forceinline__ void quantise_unit(const QuantArgs& a, int kv, int h, int cp,
+                                              const typename RawC<16>::T (&x)[NV]) {
+  using M = Mag<KIND>;
+  constexpr int VE = M::kPacked ? 8 : 4;  // elements of a vector; EW of a word
+  constexpr int EW = VE / 4;
   const barq_kv_pool& p = a.p;
-  const int t = threadIdx.x;
-  const int P = (int)p.page_size, H = (int)p.kv_heads, D = (int)p.head_dim, C = H * D;
-  const int G = C / 8, VD = D / 8, R = kThreads / G;  // R threads share a channel group
-  const int g = t % G;
-  // key maxima over the page's tokens, per channel
-  float mk[8];
+  const int lane = opaque_lane();
+  const int vd = 1 << a.vd_log2;
+  const int col = (lane & (vd - 1)) * VE;
+  const int t0 = lane >> a.vd_log2, step = kWave >> a.vd_log2;
+  const int P = (int)p.page_size, H = (int)p.kv_heads, D = (int)p.head_dim;
+  float inv[VE];      // keys: 2^-e of the columns' scale exponents e in [-127, 120] (products are exact)
+  uint32_t top[NV];   // values: the vectors' token maxima
+  bool special;
+  if (kv == 0) {
+    uint32_t m[4] = {0, 0, 0, 0};
 #pragma unroll
-  for (int e = 0; e < 8; ++e) mk[e] = 0.0f;
+    for (int i = 0; i < NV; ++i)
 #pragma unroll
-  for (int i = 0; i < NV; ++i)
+      for (int w = 0; w < 4; ++w) m[w] = M::max2(m[w], x[i][w] & M::kMask);
+    special = __builtin_amdgcn_ballot_w64(M::any_nonfinite(M::max2(M::max2(m[0], m[1]), M::max2(m[2], m[3])))) != 0;
+    if (special) {  // uniform
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mk[e] = fmaxf(mk[e], finite_abs(Regs::elem(pg.k[i], e)));
+      for (int w = 0; w < 4; ++w) {
+        m[w] = 0;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) s_red[t * 8 + e] = mk[e];
-  __syncthreads();
-  if (t < G) {
-    typename CodeVec<8>::U sc;
+        for (int i = 0; i < NV; ++i) m[w] = M::max2(m[w], M::finite(x[i][w]));
+      }
+    }
+    for (int o = vd; o < kWave; o <<= 1) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float m = s_red[t * 8 + e];
-      for (int q = 1; q < R; ++q) m = fmaxf(m, s_red[(t + q * G) * 8 + e]);
-      const int ex = group_exponent(m);
-      s_kexp[t * 8 + e] = (int8_t)ex;
+      for (int w = 0; w < 4; ++w) m[w] = M::max2(m[w], (uint32_t)__shfl_xor((int)m[w], o, kWave));
+    }
+    typename CodeVec<VE>::U sc;
+#pragma unroll
+    for (int e = 0; e < VE; ++e) {
+      const int ex = group_exponent(M::value(m[e / EW], e % EW));
+      inv[e] = __uint_as_float((uint32_t)(127 - ex) << 23);
       sc.b[e] = (uint8_t)(ex + 127);
     }
-    *(typename CodeVec<8>::Raw*)(a.c.key_scales + (int64_t)cp * C + t * 8) = sc.v;
-  }
-  __syncthreads();
-  int kex[8];
+    if (lane < vd) *(typename CodeVec<VE>::Raw*)(a.c.key_scales + ((int64_t)cp * H + h) * D + col) = sc.v;
+  } else {
+    uint32_t all = 0;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) kex[e] = s_kexp[g * 8 + e];
-  uint8_t* __restrict__ kc = a.c.codes[0] + (int64_t)cp * P * C;
-  uint8_t* __restrict__ vc = a.c.codes[1] + (int64_t)cp * P * C;
-  const int h = g / VD;
+    for (int i = 0; i < NV; ++i) {
+      top[i] = M::max2(M::max2(x[i][0] & M::kMask, x[i][1] & M::kMask), M::max2(x[i][2] & M::kMask, x[i][3] & M::kMask));
+      all = M::max2(all, top[i]);
+    }
+    special = __builtin_amdgcn_ballot_w64(M::any_nonfinite(all)) != 0;
+    if (special) {  // uniform
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+        top[i] = M::max2(M::max2(M::finite(x[i][0]), M::finite(x[i][1])), M::max2(M::finite(x[i][2]), M::finite(x[i][3])));
+    }
+    uint8_t* __restrict__ vscales = a.c.value_scales + ((int64_t)cp * P * H + h);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if constexpr (M::kPacked) top[i] = max(top[i] & 0xFFFFu, top[i] >> 16);
+      for (int o = 1; o < vd; o <<= 1) top[i] = max(top[i], (uint32_t)__shfl_xor((int)top[i], o, kWave));
+      const int ex = group_exponent(M::value(top[i], 0));
+      top[i] = (uint32_t)(127 - ex) << 23;  // 2^-e
+      if (col == 0) vscales[(uint32_t)((t0 + i * step) * H)] = (uint8_t)(ex + 127);
+    }
+  }
+  uint8_t* __restrict__ codes = a.c.codes[kv] + ((int64_t)cp * P * H + h) * D;
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int tok = t / G + i * R;
-    // value maxima over (token, head): the head's VD adjacent lanes
-    float mv = 0.0f;
+    __builtin_amdgcn_sched_barrier(0);  // one vector's floats at a time
+    typename CodeVec<VE>::U out;
+    uint32_t word[VE / 4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mv = fmaxf(mv, finite_abs(Regs::elem(pg.v[i], e)));
-    for (int o = 1; o < VD; o <<= 1) mv = fmaxf(mv, __shfl_xor(mv, o, kWave));
-    const int ve = group_exponent(mv);
-    if (g % VD == 0) a.c.value_scales[((int64_t)cp * P + tok) * H + h] = (uint8_t)(ve + 127);
-    typename CodeVec<8>::U ck, cv;
-    uint32_t wk[2], wv[2];
+    for (int q = 0; q < VE / 4; ++q) {
+      float f[4];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-      const int e = 4 * q;
-      wk[q] = e4m3_encode4(ldexpf(Regs::elem(pg.k[i], e), -kex[e]), ldexpf(Regs::elem(pg.k[i], e + 1), -kex[e + 1]),
-                           ldexpf(Regs::elem(pg.k[i], e + 2), -kex[e + 2]),
-                           ldexpf(Regs::elem(pg.k[i], e + 3), -kex[e + 3]));
-      wv[q] = e4m3_encode4(ldexpf(Regs::elem(pg.v[i], e), -ve), ldexpf(Regs::elem(pg.v[i], e + 1), -ve),
-                           ldexpf(Regs::elem(pg.v[i], e + 2), -ve), ldexpf(Regs::elem(pg.v[i], e + 3), -ve));
+      for (int k = 0; k < 4; ++k)
+        f[k] = M::value(x[i][(4 * q + k) / EW], (4 * q + k) % EW) * (kv == 0 ? inv[4 * q + k] : __uint_as_float(top[i]));
+      uint32_t nan = 0;
+      if (special) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (fabsf(f[k]) <= 3.402823466e38f) continue;
+          nan |= (((__float_as_uint(f[k]) >> 24) & 0x80u) | 0x7Fu) << (8 * k);
+          f[k] = 0.0f;
+        }
+      }
+      const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+      word[q] = (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], lo, true) | nan;
     }
-    __builtin_memcpy(ck.b, wk, 8);
-    __builtin_memcpy(cv.b, wv, 8);
-    const int64_t at = (int64_t)tok * C + g * 8;
-    *(typename CodeVec<8>::Raw*)(kc + at) = ck.v;
-    *(typename CodeVec<8>::Raw*)(vc + at) = cv.v;
+    __builtin_memcpy(out.b, word, VE);
+    *(typename CodeVec<VE>::Raw*)(codes + (uint32_t)((t0 + i * step) * H * D + col)) = out.v;
   }
 }
 
 template <int KIND, int NV>
-__global__ void __launch_bounds__(kThreads) compress_regs_kernel(const CompressArgs a) {
-  __shared__ int lds_scan[kWaves];
-  __shared__ int s_blocks[kThreads];
-  __shared__ int s_pages[kThreads];
-  __shared__ int s_cold[kThreads];
-  __shared__ int s_avail, s_top, s_slot;
-  __shared__ float s_red[kThreads * 8];
-  __shared__ int8_t s_kexp[kRegsMaxChannels];
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(NV <= 4 ? 8 : 4))) quant_blocks_kernel(const QuantArgs a) {
+  using V = typename RawC<16>::T;
+  using Bits = typename Elem<KIND>::Bits;
+  __shared__ int s_cold;
   const barq_kv_pool& p = a.p;
-  const int tid = threadIdx.x;
-  const int r = blockIdx.x;
-  const int mb = (int)p.max_blocks;
-  const int C = (int)(p.kv_heads * p.head_dim);
-  const int len = p.seq_lens[r] + a.ahead;
-  const int old_len = len - a.c.window;
-  const int jmax = min(old_len > 0 ? (int)a.div_page.div((uint32_t)old_len) : 0,
-                       min(ceil_div_fd(max(p.high_water[r], len), a.div_page), mb));
-  int32_t* row = p.block_table + (int64_t)r * mb;
+  if (a.tokens > 0 && p.ctrl[BARQ_KV_CTRL_APPEND_OK] == 0) return;  // the append was abandoned
+  const int b = (int)a.div_tiles.div(blockIdx.x);
+  const int i = (int)blockIdx.x - b * (int)a.div_tiles.d;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int nwaves = (int)blockDim.x / kWave;
+  const int P = (int)p.page_size, H = (int)p.kv_heads, D = (int)p.head_dim, mb = (int)p.max_blocks;
+  const int end = p.seq_lens[b] + a.ahead;  // the row's length after the append (or ahead of it)
+  const int len = end - a.tokens;           // positions from here on are the launch's tokens
+  const int hw = p.high_water[b];
+  const int frontier = min(end > a.c.window ? (int)a.div_page.div((uint32_t)(end - a.c.window)) : 0, mb);
+  int32_t* row = p.block_table + (int64_t)b * mb;
   int err = 0;
-  for (int j0 = 0; j0 < jmax; j0 += kThreads) {
-    const int j = j0 + tid;
-    int hot = 0, page = -1;
-    if (j < jmax) {
-      page = checked_id(row[j], p.num_pages);
-      hot = page >= 0 && (!p.page_shares || p.page_shares[page] == 0);
-    }
-    int count = 0;
-    const int k = block_exclusive_scan(hot, lds_scan, &count);
-    if (hot) {
-      s_blocks[k] = j;
-      s_pages[k] = page;
-    }
-    __syncthreads();
-    if (count == 0) continue;  // uniform
-    PageRegs<KIND, NV> pg;
-    pg.load(p, s_pages[0], C);  // in flight while the cold pages are reserved
-    if (tid == 0) {
-      const int before = atomicSub(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], count);
-      int avail = 0;
-      if ((int64_t)before > a.c.num_cold) {
-        atomicAdd(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], count);
-        err |= BARQ_KV_ERRBIT_BAD_INDEX;
+
+  const bool new_tile = i < a.nnew;
+  // Older blocks, wholly below len (compress: below the high-water mark), as far as the frontier;
+  // this tile's every kOldTiles-th of them, 64 entries (one per lane) at a time.
+  const int limit = a.tokens > 0 ? (int)a.div_page.div((uint32_t)len)
+                                 : min(ceil_div_fd(max(hw, end), a.div_page), mb);
+  int next = new_tile ? 0 : min(frontier, limit) - 1 - (i - a.nnew);
+  int first = 0, found = -1;  // the lane's hot page, of block first - lane * kOldTiles
+  uint64_t hot = 0;           // lanes whose block is still to do (the same bits in every wave)
+  for (;;) {
+    int j, hp = -1, cp = -1;
+    bool moves = false;  // a hot block that leaves the window
+    if (new_tile) {
+      j = (int)a.div_page.div((uint32_t)len) + i;
+      if (j * P >= end || j >= mb) break;
+      const int entry = row[j];
+      if (entry <= -2) {
+        if (j * P >= len) cp = checked_id(-2 - entry, a.c.num_cold);
+        if (cp < 0) err |= BARQ_KV_ERRBIT_BAD_INDEX;
       } else {
-        avail = min(max(before, 0), count);
-        if (avail < count) {
-          atomicAdd(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], count - avail);
-          err |= BARQ_KV_ERRBIT_POOL_EXHAUSTED;
+        hp = checked_id(entry, p.num_pages);
+        moves = hp >= 0 && j < frontier && (!p.page_shares || p.page_shares[hp] == 0);
+      }
+    } else {
+      while (hot == 0 && next >= 0) {
+        const int jl = next - lane * kOldTiles;
+        found = jl >= 0 ? checked_id(row[jl], p.num_pages) : -1;
+        if (found >= 0 && p.page_shares && p.page_shares[found] != 0) found = -1;
+        hot = __builtin_amdgcn_ballot_w64(found >= 0);
+        first = next;
+        next -= kOldTiles * kWave;
+      }
+      if (hot == 0) break;
+      const int l = __builtin_ctzll(hot);
+      hot &= hot - 1;
+      j = first - l * kOldTiles;
+      hp = __builtin_amdgcn_readlane(found, l);
+      moves = true;
+    }
+    if (moves) {  // uniform
+      if (threadIdx.x == 0) {
+        const int before = atomicSub(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], 1);
+        int c = -1;
+        if (before <= 0 || (int64_t)before > a.c.num_cold) {
+          atomicAdd(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], 1);
+          err |= before <= 0 ? BARQ_KV_ERRBIT_POOL_EXHAUSTED : BARQ_KV_ERRBIT_BAD_INDEX;
+        } else {
+          c = checked_id(a.c.free_cold[before - 1], a.c.num_cold);
+          if (c < 0) err |= BARQ_KV_ERRBIT_BAD_INDEX;
+        }
+        s_cold = c;
+      }
+      __syncthreads();
+      cp = s_cold;  // -1: no cold page left, the block stays hot
+    }
+#pragma unroll 1
+    for (int u = wave; u < 2 * H; u += nwaves) {  // a wave's units: heads of K, then of V
+      const int kv = u >= H ? 1 : 0, h = u - kv * H;
+      V x[NV];
+      if (cp >= 0) {
+        load_unit<KIND, NV>(a, b, kv, h, hp, j * P, len, x);
+        quantise_unit<KIND, NV>(a, kv, h, cp, x);
+      } else if (hp >= 0 && new_tile) {  // the block's new tokens into its hot page
+        const int lane = opaque_lane();
+        const int lo = max(len - j * P, 0), hi = min(end - j * P, P);
+        const int col = (lane & ((1 << a.vd_log2) - 1)) * (16 / (int)sizeof(Bits));
+        const Bits* in = (const Bits*)a.in[kv] + ((int64_t)b * a.isb + (int64_t)h * a.ish + (int64_t)(j * P - len) * a.ist);
+        Bits* page = (Bits*)(kv ? p.value_pages : p.key_pages) + ((int64_t)hp * P * H + h) * D;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          const int t = (lane >> a.vd_log2) + k * (kWave >> a.vd_log2);
+          if (t >= lo && t < hi)
+            x[k] = __builtin_nontemporal_load((const V*)(in + ((uint32_t)t * (uint32_t)a.ist + (uint32_t)col)));
+        }
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          const int t = (lane >> a.vd_log2) + k * (kWave >> a.vd_log2);
+          if (t >= lo && t < hi) *(V*)(page + (uint32_t)(t * H * D + col)) = x[k];
         }
       }
-      s_avail = avail;
-      s_top = before;
     }
-    __syncthreads();
-    const int avail = s_avail;
-    if (tid < avail) {
-      const int cp = checked_id(a.c.free_cold[s_top - 1 - tid], a.c.num_cold);
-      if (cp < 0) err |= BARQ_KV_ERRBIT_BAD_INDEX;
-      s_cold[tid] = cp;
-    }
-    __syncthreads();
-    for (int q = 0; q < avail; ++q) {
-      if (q > 0) pg.load(p, s_pages[q], C);
-      const int cp = s_cold[q];
-      if (cp >= 0) quantise_regs<KIND, NV>(a, pg, cp, s_red, s_kexp);  // uniform
-      __syncthreads();  // s_red / s_kexp reused by the next block
-    }
-    // Every thread has read every quantised hot page: map the cold pages, push the hot pages.
-    const int done = tid < avail && s_cold[tid] >= 0;
-    int n_done = 0;
-    const int pos = block_exclusive_scan(done, lds_scan, &n_done);
-    if (n_done > 0) {  // uniform
-      if (tid == 0) s_slot = atomicAdd(&p.ctrl[BARQ_KV_CTRL_FREE_TOP], n_done);
-      __syncthreads();
-      if (done) {
-        row[s_blocks[tid]] = BARQ_KV_COLD_ENTRY(s_cold[tid]);
-        const int slot = s_slot + pos;
-        if (slot < p.num_pages) p.free_pages[slot] = s_pages[tid];
+    if (moves) {
+      __syncthreads();  // every wave has read the hot page, and s_cold, before they change
+      if (threadIdx.x == 0 && cp >= 0) {
+        row[j] = BARQ_KV_COLD_ENTRY(cp);
+        const int slot = atomicAdd(&p.ctrl[BARQ_KV_CTRL_FREE_TOP], 1);
+        if (slot < p.num_pages) p.free_pages[slot] = hp;
         else err |= BARQ_KV_ERRBIT_BAD_INDEX;
       }
     }
-    __syncthreads();  // s_blocks / s_pages / s_cold reused by the next round
+    if (new_tile) break;
   }
   if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);
+}
+
+// Commit of such an append, before its blocks are written: one workgroup maps every row's new
+// blocks -- those wholly before the window at the row's new end to cold pages, the rest to hot
+// pages, each ranked in (row, block) order on its stack -- and advances the rows.  If a row passes
+// its capacity or a stack holds too few pages, nothing changes but the error bits, and
+// ctrl[BARQ_KV_CTRL_APPEND_OK] = 0 tells the launch that follows.
+struct AppendPlanArgs {
+  barq_kv_pool p;
+  ColdPtrs c;
+  int32_t batch;
+  int32_t tokens;
+  FastDiv div_page;
+};
+
+constexpr int kPlanThreads = 1024;
+
+__global__ void __launch_bounds__(kPlanThreads) append_plan_kernel(const AppendPlanArgs a) {
+  __shared__ int s_scan[2][kPlanThreads / kWave];
+  __shared__ int s_incl[2][kPlanThreads];  // rank ends of the chunk's rows: cold, hot
+  __shared__ int s_first[2][kPlanThreads];
+  __shared__ int s_bad;
+  const barq_kv_pool& p = a.p;
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1), wave = tid / kWave;
+  const int mb = (int)p.max_blocks;
+  const int top = p.ctrl[BARQ_KV_CTRL_FREE_TOP];
+  const int ctop = p.ctrl[BARQ_KV_CTRL_COLD_TOP];
+  if (tid == 0) s_bad = 0;
+  __syncthreads();
+  // pass 0 counts, pass 1 maps
+  for (int pass = 0; pass < 2; ++pass) {
+    int used[2] = {0, 0};
+    int err = 0;
+    for (int r0 = 0; r0 < a.batch; r0 += kPlanThreads) {
+      const int r = r0 + tid;
+      int n[2] = {0, 0}, first[2] = {0, 0};
+      int len = 0, hw = 0;
+      if (r < a.batch) {
+        len = p.seq_lens[r];
+        hw = p.high_water[r];
+        const int f = ceil_div_fd(hw, a.div_page);
+        const int full = ceil_div_fd(len + a.tokens, a.div_page);
+        if (full > mb) err |= BARQ_KV_ERRBIT_CAPACITY;
+        const int end = min(full, mb);
+        const int behind = len + a.tokens - a.c.window;
+        const int frontier = min(behind > 0 ? (int)a.div_page.div((uint32_t)behind) : 0, end);
+        first[0] = f;
+        n[0] = max(frontier - f, 0);
+        first[1] = max(f, frontier);
+        n[1] = max(end - first[1], 0);
+      }
+      int total[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int incl = wave_incl_scan(n[k]);
+        if (lane == kWave - 1) s_scan[k][wave] = incl;
+        __syncthreads();
+        int before = 0, all = 0;
+        for (int w = 0; w < kPlanThreads / kWave; ++w) {
+          const int t = s_scan[k][w];
+          if (w < wave) before += t;
+          all += t;
+        }
+        s_incl[k][tid] = before + incl;
+        s_first[k][tid] = first[k];
+        total[k] = all;
+      }
+      __syncthreads();
+      if (pass == 1) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          for (int q = tid; q < total[k]; q += kPlanThreads) {
+            int lo = 0, hi = kPlanThreads - 1;
+            while (lo < hi) {  // the first row whose rank end passes q
+              const int mid = (lo + hi) >> 1;
+              if (s_incl[k][mid] > q) hi = mid;
+              else lo = mid + 1;
+            }
+            const int excl = lo > 0 ? s_incl[k][lo - 1] : 0;
+            const int idx = (k == 0 ? ctop : top) - 1 - (used[k] + q);  // within the stack: pass 0 checked
+            const int id = k == 0 ? checked_id(a.c.free_cold[idx], a.c.num_cold)
+                                  : checked_id(p.free_pages[idx], p.num_pages);
+            if (id < 0) err |= BARQ_KV_ERRBIT_BAD_INDEX;
+            p.block_table[(int64_t)(r0 + lo) * mb + s_first[k][lo] + (q - excl)] =
+                k == 0 && id >= 0 ? BARQ_KV_COLD_ENTRY(id) : id;
+          }
+        }
+        if (r < a.batch) {
+          p.seq_lens[r] = len + a.tokens;
+          p.high_water[r] = max(hw, len + a.tokens);
+        }
+      }
+      used[0] += total[0];
+      used[1] += total[1];
+      __syncthreads();  // s_scan / s_incl / s_first are rewritten by the next chunk of rows
+    }
+    if (pass == 0) {
+      if (used[0] > ctop || ctop > a.c.num_cold || used[1] > top || top > p.num_pages)
+        err |= BARQ_KV_ERRBIT_POOL_EXHAUSTED;
+      if (err) atomicOr(&s_bad, err);
+      __syncthreads();
+      if (s_bad) {  // uniform
+        if (tid == 0) {
+          p.ctrl[BARQ_KV_CTRL_APPEND_OK] = 0;
+          atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], s_bad);
+        }
+        return;
+      }
+    } else {
+      if (tid == 0) {
+        p.ctrl[BARQ_KV_CTRL_COLD_TOP] = ctop - used[0];
+        p.ctrl[BARQ_KV_CTRL_FREE_TOP] = top - used[1];
+        p.ctrl[BARQ_KV_CTRL_APPEND_OK] = 1;
+      }
+      if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1326,28 +1586,62 @@ const void* compress_fn(int64_t kind, int ve) {
 }
 
 template <int KIND>
-const void* compress_regs_fn_t(int nv) {
+const void* quant_blocks_fn_t(int nv) {
   switch (nv) {
-    case 1: return (const void*)&compress_regs_kernel<KIND, 1>;
-    case 2: return (const void*)&compress_regs_kernel<KIND, 2>;
-    case 4: return (const void*)&compress_regs_kernel<KIND, 4>;
-    default: return (const void*)&compress_regs_kernel<KIND, 8>;
+    case 1: return (const void*)&quant_blocks_kernel<KIND, 1>;
+    case 2: return (const void*)&quant_blocks_kernel<KIND, 2>;
+    case 4: return (const void*)&quant_blocks_kernel<KIND, 4>;
+    default: return (const void*)&quant_blocks_kernel<KIND, 8>;
   }
 }
 
-// The register-resident compress when the geometry admits it (2-byte elements in 16-byte
-// vectors, G = kv_heads * head_dim / 8 dividing the workgroup, page_size * G / 256 vectors per
-// thread in {1, 2, 4, 8} -- 16 would not stay in registers --, head_dim / 8 a power of two up
-// to a wave), else null.
-const void* compress_regs_fn(const barq_kv_pool* p, int64_t kind, int ve) {
-  if (kind == BARQ_KV_FP32 || ve != 8) return nullptr;
-  const int64_t C = p->kv_heads * p->head_dim, G = C / 8, vd = p->head_dim / 8;
-  if (G < 1 || kThreads % G != 0 || vd > kWave || (vd & (vd - 1)) != 0 || (p->page_size * G) % kThreads != 0)
-    return nullptr;
-  const int64_t nv = p->page_size * G / kThreads;
-  if (nv != 1 && nv != 2 && nv != 4 && nv != 8) return nullptr;
-  return kind == BARQ_KV_BF16 ? compress_regs_fn_t<BARQ_KV_BF16>((int)nv)
-                              : compress_regs_fn_t<BARQ_KV_FP16>((int)nv);
+// 16-byte vectors per lane of one head of a page when quant_blocks_kernel takes the pool -- a head
+// row of a power of two of vectors, up to a wave's 64, and a head's page of 1, 2, 4 or 8 waves of
+// them -- every page, code and key-scale address aligned to its vector; else 0.
+int quant_blocks_vectors(const barq_kv_pool* p, const barq_kv_cold* c) {
+  const int64_t ve = 16 / p->elem_bytes;
+  const uint64_t bits = (uint64_t)(uintptr_t)p->key_pages | (uint64_t)(uintptr_t)p->value_pages;
+  const uint64_t cbits = (uint64_t)(uintptr_t)c->key_codes | (uint64_t)(uintptr_t)c->value_codes |
+                         (uint64_t)(uintptr_t)c->key_scales;
+  if (p->head_dim % ve || (bits & 15) || (cbits & (uint64_t)(ve - 1))) return 0;
+  const int64_t vd = p->head_dim / ve;
+  if (vd > kWave || (vd & (vd - 1)) || (p->page_size * vd) % kWave) return 0;
+  const int64_t nv = p->page_size * vd / kWave;
+  return nv == 1 || nv == 2 || nv == 4 || nv == 8 ? (int)nv : 0;
+}
+
+// Launches quant_blocks_kernel over `batch` rows: `tokens` already committed (append) or `ahead`.
+int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, int nv, int64_t batch, int64_t tokens,
+                        int64_t ahead, const void* ks, const void* vs, int64_t sb, int64_t sh, int64_t st,
+                        hipStream_t stream) {
+  QuantArgs a;
+  a.p = *pool;
+  a.c = cold_ptrs(cold);
+  a.in[0] = (const char*)ks;
+  a.in[1] = (const char*)vs;
+  a.isb = sb;
+  a.ish = sh;
+  a.ist = st;
+  a.tokens = (int32_t)tokens;
+  a.ahead = (int32_t)ahead;
+  const int64_t P = pool->page_size;
+  // `tokens` positions from anywhere in a block
+  const int64_t nnew = tokens > 0 ? (tokens + P - 2) / P + 1 : 0;
+  a.nnew = (int32_t)nnew;
+  const int64_t vd = pool->head_dim * pool->elem_bytes / 16;
+  a.vd_log2 = __builtin_ctzll((unsigned long long)vd);
+  a.div_page = FastDiv::make((uint32_t)P);
+  a.div_tiles = FastDiv::make((uint32_t)(nnew + kOldTiles));
+  const int64_t tiles = batch * (nnew + kOldTiles);
+  if (tiles > kI32Max) return BARQ_KV_ERR_INVALID;
+  const void* fn = cold->element_type == BARQ_KV_BF16   ? quant_blocks_fn_t<BARQ_KV_BF16>(nv)
+                   : cold->element_type == BARQ_KV_FP16 ? quant_blocks_fn_t<BARQ_KV_FP16>(nv)
+                                                        : quant_blocks_fn_t<BARQ_KV_FP32>(nv);
+  const int threads = kWave * (int)std::min<int64_t>(16, 2 * pool->kv_heads);
+  void* args[] = {&a};
+  return hipLaunchKernel(fn, dim3((uint32_t)tiles), dim3((uint32_t)threads), args, 0, stream) == hipSuccess
+             ? BARQ_KV_OK
+             : BARQ_KV_ERR_LAUNCH;
 }
 
 template <int KIND>
@@ -1386,6 +1680,8 @@ int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t 
                     void* stream) {
   if (!cold_ok(pool, cold) || batch < 0 || batch > pool->max_batch) return BARQ_KV_ERR_INVALID;
   if (batch == 0) return BARQ_KV_OK;
+  if (const int nv = quant_blocks_vectors(pool, cold))
+    return launch_quant_blocks(pool, cold, nv, batch, 0, ahead, nullptr, nullptr, 0, 0, 0, (hipStream_t)stream);
   CompressArgs a;
   a.p = *pool;
   a.c = cold_ptrs(cold);
@@ -1401,8 +1697,7 @@ int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t 
   int ve = eb == 2 ? 8 : 4;
   while (ve > 1 && (D % ve || (bits & (uint64_t)(ve * eb - 1)) || (cbits & (uint64_t)(ve - 1)))) ve >>= 1;
   a.div_groups = FastDiv::make((uint32_t)(pool->kv_heads * D / ve));
-  const void* fn = compress_regs_fn(pool, cold->element_type, ve);
-  return launch(fn ? fn : compress_fn(cold->element_type, ve), dim3((uint32_t)batch), &a, (hipStream_t)stream);
+  return launch(compress_fn(cold->element_type, ve), dim3((uint32_t)batch), &a, (hipStream_t)stream);
 }
 
 // The update in two launches -- compress for the lengths the rows reach, then
@@ -1430,6 +1725,33 @@ int resident_tiles(const void* fn, int slot) {
     cached[slot][dev].store(v, std::memory_order_relaxed);
   }
   return v;
+}
+
+// barq_kv_update_cold's BARQ_KV_QUANT_DIRECT append.
+int append_direct(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* key_states, const void* value_states,
+                  int64_t batch, int64_t tokens, int64_t stride_b, int64_t stride_h, int64_t stride_t, void* stream) {
+  if (!cold_ok(pool, cold) || batch < 0 || batch > pool->max_batch || tokens < 0) return BARQ_KV_ERR_INVALID;
+  if (tokens > pool->max_blocks * pool->page_size) return BARQ_KV_ERR_INVALID;
+  if (batch == 0 || tokens == 0) return BARQ_KV_OK;
+  if (!key_states || !value_states || stride_b < 0 || stride_h < 0 || stride_t < 0) return BARQ_KV_ERR_INVALID;
+  const int nv = quant_blocks_vectors(pool, cold);
+  const int64_t eb = pool->elem_bytes;
+  const uint64_t bits = (uint64_t)(uintptr_t)key_states | (uint64_t)(uintptr_t)value_states |
+                        (uint64_t)(stride_b * eb) | (uint64_t)(stride_h * eb) | (uint64_t)(stride_t * eb);
+  // lane offsets within a block of the input fit 32 bits
+  if (nv == 0 || (bits & 15) || stride_t > kI32Max / (pool->page_size * eb)) return BARQ_KV_ERR_UNSUPPORTED;
+  AppendPlanArgs a;
+  a.p = *pool;
+  a.c = cold_ptrs(cold);
+  a.batch = (int32_t)batch;
+  a.tokens = (int32_t)tokens;
+  a.div_page = FastDiv::make((uint32_t)pool->page_size);
+  void* args[] = {&a};
+  if (hipLaunchKernel((const void*)&append_plan_kernel, dim3(1), dim3(kPlanThreads), args, 0,
+                      (hipStream_t)stream) != hipSuccess)
+    return BARQ_KV_ERR_LAUNCH;
+  return launch_quant_blocks(pool, cold, nv, batch, tokens, 0, key_states, value_states, stride_b, stride_h, stride_t,
+                             (hipStream_t)stream);
 }
 
 int update_cold_fused(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* ks, const void* vs,
@@ -1561,7 +1883,16 @@ int barq_kv_update_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, cons
                         int64_t seq_out, int64_t osb, int64_t osh, int64_t oss, int64_t flags,
                         void* stream) {
   if (!cold_ok(pool, cold)) return BARQ_KV_ERR_INVALID;
-  if (flags & ~(int64_t)(BARQ_KV_SEQ_FROM_DEVICE | BARQ_KV_NO_COMPRESS)) return BARQ_KV_ERR_INVALID;
+  if (flags & ~(int64_t)(BARQ_KV_SEQ_FROM_DEVICE | BARQ_KV_NO_COMPRESS | BARQ_KV_QUANT_DIRECT)) return BARQ_KV_ERR_INVALID;
+  if (flags & BARQ_KV_QUANT_DIRECT) {
+    if (flags & BARQ_KV_NO_COMPRESS) return BARQ_KV_ERR_INVALID;
+    if (seq_out < 0 || seq_out > pool->max_blocks * pool->page_size || (seq_out > 0 && (!key_out || !value_out)))
+      return BARQ_KV_ERR_INVALID;
+    const int rc = append_direct(pool, cold, key_states, value_states, batch, tokens, stride_b, stride_h, stride_t, stream);
+    return rc != BARQ_KV_OK ? rc
+                            : barq_kv_gather_cold(pool, cold, key_out, value_out, batch, seq_out, osb, osh, oss,
+                                                  flags & BARQ_KV_SEQ_FROM_DEVICE, stream);
+  }
   const int fused = update_cold_fused(pool, cold, key_states, value_states, batch, tokens, stride_b, stride_h,
                                       stride_t, key_out, value_out, seq_out, osb, osh, oss, flags, stream);
   if (fused >= 0) return fused;

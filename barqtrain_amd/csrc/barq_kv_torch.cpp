@@ -297,6 +297,23 @@ void pool_compress_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, 
   check_status(barq_kv_compress(&p, &c, batch, current_stream(pool[0])), "pool_compress_");
 }
 
+// Append of any number of tokens, quantising what passes the window as it is stored; false (nothing
+// launched) when the pool or the states have a form the kernels do not take.
+bool pool_append_cold_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
+                       at::Tensor key_states, at::Tensor value_states) {
+  barq_kv_pool p = pool_from(pool);
+  barq_kv_cold c = cold_from(p, pool[0], cold, window);
+  check_states(p, pool[0], key_states, value_states);
+  c10::DeviceGuard guard(pool[0].device());
+  const int rc = barq_kv_update_cold(&p, &c, key_states.data_ptr(), value_states.data_ptr(), key_states.size(0),
+                                     key_states.size(2), key_states.stride(0), key_states.stride(1),
+                                     key_states.stride(2), nullptr, nullptr, 0, 0, 0, 0, BARQ_KV_QUANT_DIRECT,
+                                     current_stream(pool[0]));
+  if (rc == BARQ_KV_ERR_UNSUPPORTED) return false;
+  check_status(rc, "pool_append_cold_");
+  return true;
+}
+
 void pool_gather_cold(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
                       at::Tensor key_out, at::Tensor value_out, int64_t batch, int64_t seq_out, int64_t flags) {
   barq_kv_pool p = pool_from(pool);
@@ -567,6 +584,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pool_select_rows_", &pool_select_rows_, "Rows become selected rows, sharing their full pages");
   m.def("pool_cold_reset_", &pool_cold_reset_, "Every page of a pool's fp8 cold store free");
   m.def("pool_compress_", &pool_compress_, "Quantise blocks behind the residual window into the cold store");
+  m.def("pool_append_cold_", &pool_append_cold_, "Append tokens, quantising past the residual window as they are stored");
   m.def("pool_gather_cold", &pool_gather_cold, "Materialise rows of a pool with a cold store, dequantising");
   m.def("pool_update_cold_", &pool_update_cold_, "Append, compress, materialise (pool with a cold store)");
   m.def("pool_free_rows_cold_", &pool_free_rows_cold_, "Return rows' hot and cold pages");

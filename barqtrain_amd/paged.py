@@ -644,6 +644,8 @@ class QuantPagePool(PagePool):
             # Every chunk's capacity, hot-page and cold-page needs are checked up front, so an
             # append that cannot finish raises before its first chunk changes anything.
             self._check_chunked(batch, tokens, max_length)
+            if self.on_gpu and self._append_direct(self.tensors, slice(0, batch), key_states, value_states):
+                return
             for s0 in range(0, tokens, self.chunk):
                 self.append(key_states[:, :, s0:s0 + self.chunk], value_states[:, :, s0:s0 + self.chunk],
                             max_length)
@@ -655,9 +657,36 @@ class QuantPagePool(PagePool):
         k, v = self._compatible_pair(key_states, value_states)
         ops = self._ops()
         ops.pool_append_(self.tensors, k, v)
-        ops.pool_compress_(self.tensors, self.cold_tensors, self.window, batch)
+        if moved:  # else no block leaves the window: no compress launch
+            ops.pool_compress_(self.tensors, self.cold_tensors, self.window, batch)
         self._advance(batch, tokens, need)
         self._quantised(batch, frontier, moved)
+
+    def _append_direct(self, tensors: list[torch.Tensor], rows: slice, key_states: torch.Tensor,
+                       value_states: torch.Tensor) -> bool:
+        """A checked append of `rows` (the rows of `tensors`) in one go, blocks past the window
+        quantised from the states themselves (BARQ_KV_QUANT_DIRECT): no chunks, and hot pages only
+        for what stays hot.  False, nothing changed, when the free hot pages do not cover those at
+        once (chunks also use the pages that quantised blocks return) or the kernels do not take
+        the geometry."""
+        tokens, P = key_states.shape[2], self.page_size
+        lens, hw, cold = self.lens[rows], self.hw[rows], self.cold_blocks[rows]
+        ends = lens + tokens
+        frontier = np.maximum(ends - self.window, 0) // P
+        mapped = -(-hw // P)
+        last = -(-ends // P)
+        if int(np.maximum(last - np.maximum(mapped, frontier), 0).sum()) > self.free_count:
+            return False
+        k, v = self._compatible_pair(key_states, value_states)
+        if not self._ops().pool_append_cold_(tensors, self.cold_tensors, self.window, k, v):
+            return False
+        moved = int(np.maximum(frontier - cold, 0).sum())
+        self.free_count += moved - int(np.maximum(last - mapped, 0).sum())
+        self.cold_free -= moved
+        np.maximum(cold, frontier, out=cold)
+        lens += tokens
+        np.maximum(hw, lens, out=hw)
+        return True
 
     def _check_chunked(self, batch: int, tokens: int, max_length: Optional[int],
                        rows: Optional[np.ndarray] = None) -> None:
@@ -684,6 +713,14 @@ class QuantPagePool(PagePool):
             self.cold_free = int(self.ctrl[CTRL_COLD_TOP].item())
             self.cold_exact = True
         free, cold_free, P = self.free_count, self.cold_free, self.page_size
+        # Rows in their usual state -- no stale blocks past their length, everything before the
+        # window quantised -- hold at most `peak` hot blocks during a chunk: when the stacks cover
+        # that and the blocks that end up quantised, every chunk fits.
+        if (hw <= lens).all() and (cold >= np.maximum(lens - self.window, 0) // P).all():
+            peak = -(-(self.window + self.chunk) // P) + 2
+            more = np.maximum(peak - (-(-hw // P) - cold), 0).sum()
+            if more <= free and (np.maximum(np.maximum(lens + tokens - self.window, 0) // P - cold, 0)).sum() <= cold_free:
+                return
         for s0 in range(0, tokens, self.chunk):
             t = min(self.chunk, tokens - s0)
             end = np.minimum(-(-(lens + t) // P), self.max_blocks)
@@ -810,6 +847,9 @@ class QuantPagePool(PagePool):
         P = self.page_size
         for i, row in enumerate(rows):
             one = t[:2] + [t[2][row:row + 1], t[3][row:row + 1], t[4][row:row + 1]] + t[5:]
+            if (self.on_gpu and tokens > self.chunk
+                    and self._append_direct(one, slice(row, row + 1), k[i:i + 1], v[i:i + 1])):
+                continue
             for s0 in range(0, tokens, self.chunk):
                 n = min(self.chunk, tokens - s0)
                 start = int(self.lens[row])

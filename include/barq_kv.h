@@ -56,12 +56,14 @@ extern "C" {
 #define BARQ_KV_ERR_LAUNCH 2  /* the HIP runtime refused a launch */
 #define BARQ_KV_ERR_SCRATCH 3 /* the request needs more than the library's static scratch
                                  (BARQ_KV_SCRATCH_BYTES per GPU); use the workspace variant */
+#define BARQ_KV_ERR_UNSUPPORTED 4 /* valid, but of a form this entry point has no kernel for */
 
 /* Words of barq_kv_pool.ctrl.  Counters sit on lines of their own; all counters are 0 between
    launches. */
 #define BARQ_KV_CTRL_FREE_TOP 0 /* number of entries of free_pages that are free pages */
 #define BARQ_KV_CTRL_ERRORS 1   /* sticky error bits below, set by kernels, cleared by reset */
 #define BARQ_KV_CTRL_COLD_TOP 2 /* number of entries of a cold store's free_cold that are free */
+#define BARQ_KV_CTRL_APPEND_OK 3 /* the running BARQ_KV_QUANT_DIRECT append committed (1) or was abandoned (0) */
 #define BARQ_KV_CTRL_ARRIVED 32 /* tile arrival counter of the running launch */
 #define BARQ_KV_CTRL_SUBCOUNTER0 64       /* first of the arrival sub-counters ... */
 #define BARQ_KV_CTRL_SUBCOUNTER_STRIDE 64 /* ... one per 256 bytes ... */
@@ -372,8 +374,8 @@ int barq_kv_cold_reset(const barq_kv_pool* pool, const barq_kv_cold* cold, void*
  * Rows [0, batch): every hot block wholly before the residual window is quantised into a cold
  * page taken from free_cold and its hot page returns to free_pages (in no fixed order).  A block
  * finding no cold page stays hot and sets BARQ_KV_ERRBIT_POOL_EXHAUSTED; a hot page another
- * block shares (page_shares) stays hot.  One workgroup per row; rows without such a block exit
- * at once, so it can run after every append (and inside a captured graph).
+ * block shares (page_shares) stays hot.  Rows without such a block cost next to nothing, so it can
+ * run after every append (and inside a captured graph).
  */
 int barq_kv_compress(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, void* stream);
 
@@ -396,8 +398,21 @@ int barq_kv_gather_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, void
  * gather returns their dequantised values).
  * flags: BARQ_KV_SEQ_FROM_DEVICE as for the gather; BARQ_KV_NO_COMPRESS skips the compress launch
  * -- for a caller that knows no row's block leaves the window in this call (every page_size-th
- * token). */
+ * token).
+ * BARQ_KV_QUANT_DIRECT: any number of tokens in one go -- new blocks wholly before the residual
+ * window at their row's new end are quantised straight from the input and never take a hot page, so
+ * a row needs ceil(window / page_size) + 1 of them whatever the prompt -- and then the gather, if
+ * seq_out > 0 (key_out and value_out may be null when it is 0).  The cache reads the same
+ * afterwards; cold and hot pages of new blocks come off their stacks in (row, block) order.  All or
+ * nothing: when a row would pass its capacity or a stack holds too few pages for the new blocks, no
+ * row changes and the error bits say why.  (A block that was hot before and finds no cold page stays
+ * hot, as in barq_kv_compress.)  Hot pages must have one holder, as a selection over pools with cold
+ * stores leaves them.  Takes pools whose head rows are a power of two of 16-byte vectors, up to 64,
+ * with 64, 128, 256 or 512 vectors to a head's page, and addresses and strides that are multiples
+ * of 16 bytes (codes and key scales: 16 / elem_bytes); others return BARQ_KV_ERR_UNSUPPORTED with
+ * nothing launched. */
 #define BARQ_KV_NO_COMPRESS 4
+#define BARQ_KV_QUANT_DIRECT 8
 int barq_kv_update_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* key_states,
                         const void* value_states, int64_t batch, int64_t tokens, int64_t stride_b,
                         int64_t stride_h, int64_t stride_t, void* key_out, void* value_out,
