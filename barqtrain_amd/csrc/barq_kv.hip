@@ -60,6 +60,10 @@ constexpr int64_t kLargeLaunchTiles = 1536;
 // Stream-kernel tiles (five-wave workgroups) resident on one CU at once.
 constexpr int64_t kResidentTilesPerCU = 4;
 
+// Rows kernel: tiles resident on one CU (32 waves), and a tile's own cost in slots.
+constexpr int64_t kRowsResidentTilesPerCU = 6;
+constexpr int64_t kRowsTileSlots = 2;
+
 template <int VB>
 struct VecT;
 template <>
@@ -232,6 +236,8 @@ struct StreamArgs {
   FastDiv div_page;  // by page_size
   FastDiv div_chunks;
   FastDiv div_pieces;  // by tail pieces per (row, K or V)
+  int32_t slots;       // rows kernel: wave loads per copy wave
+  FastDiv div_loads;   // rows kernel: by wave loads per page
 };
 
 // LPP > 0: hv = 64 * LPP (LPP = 1, 2 or 4) and offsets within a page, a row's output and a row's
@@ -927,6 +933,197 @@ __global__ void __launch_bounds__(kStreamThreads) lean_known_kernel(const Stream
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Gather / update for token rows that are not whole runs of 64 vectors (2 KV heads x 64 in two
+// bytes: 16 vectors; 5 x 128: 80), batch <= 64: a page is page_size * hv / 64 = NL wave loads of
+// 1 KiB ("slots"), so a slot's page, block and first position are wave-uniform whatever the row.  A
+// copy wave takes `slots` consecutive slots of a (row, K or V) stream, all its loads in flight
+// before its first store; the host picks the count that gives every CU work -- a row of 256 bytes
+// cut into 64 KiB tiles filled fewer than the 256 CUs (24 rows of 1024 positions, 25 MB: 240 tiles,
+// 10.6 us; 768 of these, 7.9 us, ~4 us of it the launch and its two round trips).  Metadata and commit as in the lean kernels: from the arguments (KNOWN),
+// or read by every copy wave before the tile arrives.
+//
+// A wave whose slots all hold old positions, or all new tokens, moves them without a branch or a
+// per-lane decision; the others (a row's end, padding, an unmapped page) decide per vector.  COL:
+// hv divides 64, a lane's column is the same in every slot.
+// ---------------------------------------------------------------------------------------------
+template <int NU, bool KNOWN, bool COL>
+__device__ __forceinline__ void lean_rows_body(const StreamArgs& a, const KnownState* ks) {
+  using V = typename VecT<16>::T;
+  const barq_kv_pool& p = a.pool;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int lane = (int)(threadIdx.x & (kWave - 1));
+  const int bid = (int)blockIdx.x;
+  const int kv = bid & 1;
+  const int rest = bid >> 1;
+  const int b = (int)a.div_chunks.div((uint32_t)rest);
+  const int c = rest - b * (int)a.div_chunks.d;
+  const int T = a.tokens;
+  const int P = (int)p.page_size;
+  const int mb = (int)p.max_blocks;
+  const int NL = (int)a.div_loads.d;
+  const bool committing = T > 0 && a.commit_in_kernel;
+
+  if (wave == 0) {
+    if (!committing) return;
+    if constexpr (KNOWN) {
+      if (bid != 0) return;
+      const int clen = lane < a.batch ? ks->len[lane] : 0;
+      const int chw = lane < a.batch ? ks->hw[lane] : 0;
+      const int news = wave_sum(lane < a.batch ? new_blocks(clen, chw, T, mb, a.div_page).count : 0);
+      const int fidx = ks->top - 1 - lane;
+      const int cfree = news > 0 && fidx >= 0 ? p.free_pages[fidx] : -1;
+      commit_from_lanes(p, a.batch, T, a.seq_out, a.div_page, clen, chw, ks->top, cfree);
+    } else {
+      __syncthreads();  // every copy wave of the tile holds the metadata it uses
+      arrive_and_commit(p, a.nsub, a.batch, T, a.seq_out, a.div_page);
+    }
+    return;
+  }
+
+  // Copy wave: slots [slot0, slot0 + a.slots) of the stream, pages pg0 .. (one per lane).
+  const int len = KNOWN ? ks->len[b] : p.seq_lens[b];
+  const int hw = KNOWN ? ks->hw[b] : p.high_water[b];
+  const int slot0 = (c * kCopyWaves + wave - 1) * a.slots;
+  const int pg0 = (int)a.div_loads.div((uint32_t)slot0);
+  const int pgn = (int)a.div_loads.div((uint32_t)(slot0 + a.slots - 1)) - pg0 + 1;
+  const int blk = pg0 + lane;
+  const bool mine = lane < pgn && blk < mb;
+  const int entry = mine ? p.block_table[(int64_t)b * mb + blk] : -1;
+  int S = a.seq_out;
+  if (a.seq_from_device && (pg0 + pgn) * P > min(len + T, S))
+    S = min(wave_max(lane < a.batch ? p.seq_lens[lane] + T : 0), S);
+  const NewBlocks nb = new_blocks(len, hw, T, mb, a.div_page);
+  int page = blk < nb.first ? checked_page(entry, p.num_pages) : -1;
+  if (nb.count > 0 && pg0 < nb.first + nb.count && pg0 + pgn > nb.first) {
+    const int top = KNOWN ? ks->top : p.ctrl[BARQ_KV_CTRL_FREE_TOP];
+    const int rl = lane < b ? (KNOWN ? ks->len[lane] : p.seq_lens[lane]) : 0;
+    const int rh = lane < b ? (KNOWN ? ks->hw[lane] : p.high_water[lane]) : 0;
+    const int base = wave_sum(lane < b ? new_blocks(rl, rh, T, mb, a.div_page).count : 0);
+    const int idx = top - 1 - (base + blk - nb.first);
+    if (mine && blk >= nb.first && blk < nb.first + nb.count && idx >= 0)
+      page = checked_page(p.free_pages[idx], p.num_pages);
+  }
+  if (!KNOWN && committing) {
+    __builtin_amdgcn_s_waitcnt(0);  // the metadata loads have returned before the tile arrives
+    __syncthreads();
+  }
+  // slots of this wave that reach below S
+  const int lo = pg0 * P;
+  if (lo >= S) return;
+  const int hv = a.hv;
+  const int pos_per_slot = COL ? (int)a.div_hv.div(kWave) : 0;  // COL: 64 / hv
+  // slot i: first position and its page's index among the wave's pages
+  const auto slot_page = [&](int i) { return (int)a.div_loads.div((uint32_t)(slot0 + i)) - pg0; };
+  const auto slot_part = [&](int i, int pk) { return slot0 + i - (pg0 + pk) * NL; };
+  const auto first_pos = [&](int pk, int part) {  // of the slot
+    return (pg0 + pk) * P + (COL ? part * pos_per_slot : (int)a.div_hv.div((uint32_t)(part * kWave)));
+  };
+  int n = 0;  // live slots
+  for (int i = 0; i < NU; ++i) {
+    if (i >= a.slots) break;
+    const int pk = slot_page(i);
+    if (first_pos(pk, slot_part(i, pk)) >= S) break;
+    n = i + 1;
+  }
+  if (n == 0) return;
+  const int pk_last = slot_page(n - 1);
+  const int part_last = slot_part(n - 1, pk_last);
+  const int pk_0 = 0;
+  const int beg = first_pos(pk_0, slot_part(0, 0));
+  const int end = min((pg0 + pk_last) * P + (int)a.div_hv.div((uint32_t)(part_last * kWave + kWave - 1)) + 1, S);
+  const bool mapped = __builtin_amdgcn_ballot_w64(lane <= pk_last && page < 0) == 0;
+  const bool all_old = mapped && (end <= len || (beg >= len + T && end <= hw));
+  const bool all_new = mapped && beg >= len && end <= len + T;
+
+  // lane geometry; COL: the same in every slot
+  const uint32_t oss = (uint32_t)a.out_ss, ist = (uint32_t)a.in_st;
+  const int ctok = COL ? (int)a.div_hv.div((uint32_t)lane) : 0;
+  const auto lane_at = [&](int part, int& tok, uint32_t& oh, uint32_t& ih) {  // position within the page, head offsets
+    const int v = COL ? lane : part * kWave + lane;
+    const int t = COL ? ctok : (int)a.div_hv.div((uint32_t)v);
+    const int hvi = v - t * hv;
+    const int h = (int)a.div_vr.div((uint32_t)hvi);
+    const uint32_t x = (uint32_t)(hvi - h * (int)a.div_vr.d) * 16u;
+    oh = (uint32_t)h * (uint32_t)a.out_sh + x;
+    ih = (uint32_t)h * (uint32_t)a.in_sh + x;
+    tok = COL ? part * pos_per_slot + t : t;
+  };
+  const char* in_row = (kv ? a.in_v : a.in_k) + (int64_t)b * a.in_sb;
+  char* out_row = (kv ? a.out_v : a.out_k) + (int64_t)b * a.out_sb;
+  char* pages = (char*)(kv ? p.value_pages : p.key_pages);
+  V val[NU];
+  if (all_old) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int i = min(u, n - 1);  // slots past the wave's repeat its last (a cache hit)
+      const int pk = slot_page(i);
+      const int64_t pb = (int64_t)__builtin_amdgcn_readlane(page, pk) * a.page_bytes + slot_part(i, pk) * (kWave * 16);
+      val[u] = ld_stream<V>((pages + pb) + (uint32_t)(lane * 16));
+    }
+  } else if (all_new) {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int i = min(u, n - 1);
+      const int pk = slot_page(i);
+      int tok;
+      uint32_t oh, ih;
+      lane_at(slot_part(i, pk), tok, oh, ih);
+      const int s = min((pg0 + pk) * P + tok, end - 1);  // lanes past the extent repeat the last position
+      val[u] = ld_stream<V>(in_row + ((int64_t)(s - len) * ist + ih));
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      val[u] = zero_vec<V>();
+      if (u < n) {
+        const int pk = slot_page(u), part = slot_part(u, pk);
+        int tok;
+        uint32_t oh, ih;
+        lane_at(part, tok, oh, ih);
+        const int s = (pg0 + pk) * P + tok;
+        const int pg = __builtin_amdgcn_readlane(page, pk);
+        if (s < S) {
+          if ((unsigned)(s - len) < (unsigned)T) {
+            val[u] = ld_stream<V>(in_row + ((int64_t)(s - len) * ist + ih));
+          } else if (s < hw && pg >= 0) {
+            val[u] = ld_stream<V>(pages + (int64_t)pg * a.page_bytes + (uint32_t)((part * kWave + lane) * 16));
+          }
+        }
+      }
+    }
+  }
+  const bool paced = gridDim.x > kKnownBackToBackTiles;
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    if (u < n) {
+      const int pk = slot_page(u), part = slot_part(u, pk);
+      int tok;
+      uint32_t oh, ih;
+      lane_at(part, tok, oh, ih);
+      const int s = (pg0 + pk) * P + tok;
+      if (paced) wait_vm<0>();
+      if (s < S) {
+        st_stream<V>((out_row + (int64_t)(pg0 + pk) * P * a.out_ss) + ((uint32_t)tok * oss + oh), val[u]);
+        if (!all_old && (unsigned)(s - len) < (unsigned)T) {
+          const int pg = __builtin_amdgcn_readlane(page, pk);
+          if (pg >= 0) *(V*)((pages + (int64_t)pg * a.page_bytes) + (uint32_t)((part * kWave + lane) * 16)) = val[u];
+        }
+      }
+    }
+  }
+}
+
+template <int NU, bool COL>
+__global__ void __launch_bounds__(kStreamThreads) lean_rows_kernel(const StreamArgs a) {
+  lean_rows_body<NU, false, COL>(a, nullptr);
+}
+
+template <int NU, bool COL>
+__global__ void __launch_bounds__(kStreamThreads) lean_rows_known_kernel(const StreamArgs a, const KnownState ks) {
+  lean_rows_body<NU, true, COL>(a, &ks);
 }
 
 // Balanced lean tiles: lean_stream_kernel's work for chunks that start anywhere in a page.
@@ -1800,6 +1997,24 @@ int launch_known_kernel(int nu, int lpp, dim3 grid, StreamArgs* arg, const Known
                                                                                       : BARQ_KV_ERR_LAUNCH;
 }
 
+int launch_rows_kernel(int nu, bool col, dim3 grid, StreamArgs* arg, const KnownState* known, hipStream_t stream) {
+  const void* fn = nullptr;
+#define BARQ_ROWS_CASE(NU)                                                                                      \
+  fn = known ? (col ? (const void*)&lean_rows_known_kernel<NU, true> : (const void*)&lean_rows_known_kernel<NU, false>) \
+             : (col ? (const void*)&lean_rows_kernel<NU, true> : (const void*)&lean_rows_kernel<NU, false>);
+  switch (nu) {
+    case 2: BARQ_ROWS_CASE(2) break;
+    case 4: BARQ_ROWS_CASE(4) break;
+    default: BARQ_ROWS_CASE(8) break;
+  }
+#undef BARQ_ROWS_CASE
+  KnownState ks{};
+  if (known) ks = *known;
+  void* args[] = {arg, &ks};
+  return hipLaunchKernel(fn, grid, dim3(kStreamThreads), args, 0, stream) == hipSuccess ? BARQ_KV_OK
+                                                                                      : BARQ_KV_ERR_LAUNCH;
+}
+
 BARQ_DEFINE_VB_LAUNCH(dense_append_kernel, DenseArgs)
 BARQ_DEFINE_VB_LAUNCH(copy_rows_kernel, CopyArgs)
 BARQ_DEFINE_VB_LAUNCH(select_build_kernel, SelectArgs)
@@ -1882,6 +2097,36 @@ int run_stream(const barq_kv_pool* pool, const void* ks, const void* vs, int64_t
     }
   }
 
+  // Rows kernel: a gather launch the wave-uniform mapping does not take, in 16-byte vectors, whose
+  // pages are whole wave loads (offsets within a page, its output and its input positions fit 32 bits).
+  // Slots per copy wave: the launch ends with the CUs that hold the most tiles, so the count with the
+  // least work on those -- tiles times slots, a tile's own cost (metadata, its first round trip)
+  // counted as kRowsTileSlots more -- while the tiles are resident at once, else 8.  (24 rows of
+  // 1024 x 256 B, K and V: 2 / 3 / 4 / 8 slots, 6 / 4.1 / 3 / 1.5 tiles a CU, 9.6 / 8.7 / 8.0 / 8.5 us.)
+  int64_t row_slots = 0, row_chunks = 0;
+  const auto block32 = [&](int64_t stride, int64_t head_span) {
+    return stride >= 0 && stride <= kI32Max && P * stride + head_span <= kI32Max;
+  };
+  if (gather && !fast && vb == 16 && batch <= kWave && ncu > 0 && (P * hv) % kWave == 0 && P * hv / kWave <= kI32Max / 64 &&
+      P * tok_bytes <= kI32Max && osh * eb <= kI32Max && block32(oss * eb, head_span_out) &&
+      (tokens == 0 || (sh * eb <= kI32Max && block32(st * eb, head_span_in)))) {
+    const int64_t loads = P * hv / kWave;                      // per page
+    const int64_t stream_slots = (seq_out + P - 1) / P * loads;
+    int64_t best = INT64_MAX;
+    for (int64_t k = 1; k <= 8; ++k) {
+      const int64_t chunks_k = (stream_slots + kCopyWaves * k - 1) / (kCopyWaves * k);
+      const int64_t per_cu = (2 * batch * chunks_k + ncu - 1) / ncu;
+      if (per_cu <= kRowsResidentTilesPerCU || k == 8) {
+        if (per_cu * (k + kRowsTileSlots) < best) {
+          best = per_cu * (k + kRowsTileSlots);
+          row_slots = k;
+          row_chunks = chunks_k;
+        }
+      }
+    }
+    if (stream_slots + kCopyWaves * row_slots > kI32Max / 2 || 2 * batch * row_chunks > kI32Max) row_slots = 0;
+  }
+
   // Positions per tile: whole pages, about kTileTargetBytes of each of K and V.
   int64_t pages_per_tile = kTileTargetBytes / (P * tok_bytes);
   if (pages_per_tile < 1) pages_per_tile = 1;
@@ -1952,13 +2197,26 @@ int run_stream(const barq_kv_pool* pool, const void* ks, const void* vs, int64_t
   hipStream_t s = (hipStream_t)stream;
   // Launches with more tiles than the CUs hold at once take the kernel built for several rounds.
   const bool rounds = fast && ncu > 0 && grid > kResidentTilesPerCU * ncu;
-  // The caller's row state in the arguments: page-aligned lean launches of an append and gather
-  // whose extent is given (the per-call path of an eager caller).
-  if (known && lean_ppt > 0 && lean_m == 0 && tokens > 0 && a.commit_in_kernel && !a.seq_from_device)
+  int rc;
+  if (row_slots > 0) {
+    a.slots = (int32_t)row_slots;
+    a.div_loads = FastDiv::make((uint32_t)(P * hv / kWave));
+    a.div_chunks = FastDiv::make((uint32_t)row_chunks);
+    const int64_t row_grid = 2 * batch * row_chunks;
+    a.nsub = (int32_t)std::min<int64_t>(row_grid, BARQ_KV_CTRL_SUBCOUNTERS);
+    const KnownState* k = known && tokens > 0 && a.commit_in_kernel && !a.seq_from_device ? known : nullptr;
+    rc = launch_rows_kernel(row_slots <= 2 ? 2 : row_slots <= 4 ? 4 : 8, kWave % hv == 0, dim3((uint32_t)row_grid), &a,
+                            k, s);
+  } else if (known && lean_ppt > 0 && lean_m == 0 && tokens > 0 && a.commit_in_kernel && !a.seq_from_device) {
+    // The caller's row state in the arguments: page-aligned lean launches of an append and gather
+    // whose extent is given (the per-call path of an eager caller).
     return launch_known_kernel((int)lean_nu, (int)lpp, dim3((uint32_t)grid), &a, known, s);
-  int rc = lean_ppt > 0 ? (lean_m > 0 ? launch_lean_kernel<true>((int)lean_nu, (int)lpp, dim3((uint32_t)grid), &a, s)
-                                      : launch_lean_kernel<false>((int)lean_nu, (int)lpp, dim3((uint32_t)grid), &a, s))
-                        : launch_stream_kernel(vb, fast ? (int)(hv / 64) : 0, rounds, dim3((uint32_t)grid), &a, s);
+  } else if (lean_ppt > 0) {
+    rc = lean_m > 0 ? launch_lean_kernel<true>((int)lean_nu, (int)lpp, dim3((uint32_t)grid), &a, s)
+                    : launch_lean_kernel<false>((int)lean_nu, (int)lpp, dim3((uint32_t)grid), &a, s);
+  } else {
+    rc = launch_stream_kernel(vb, fast ? (int)(hv / 64) : 0, rounds, dim3((uint32_t)grid), &a, s);
+  }
   if (rc != BARQ_KV_OK) return rc;
   if (tokens > 0 && !a.commit_in_kernel) {
     barq_kv_pool pc = *pool;
