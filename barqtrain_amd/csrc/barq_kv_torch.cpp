@@ -386,56 +386,87 @@ void pool_select_rows_cold_(std::vector<std::vector<at::Tensor>> pools, std::vec
                "pool_select_rows_cold_");
 }
 
-// One decode-step call of PagePool.update / append with its host planning in C++: the capacity
-// and free-page checks of the host shadow (int64 arrays lens / hw, updated in place on success),
-// output allocation and the launch.  handle: pool_group of this one pool; pages: its key_pages
-// (device, dtype).  Returns (key_out, value_out, pages taken); pages taken < 0 when the call must
-// take the checked Python path instead, which raises the exact error (-1: capacity exceeded, -2:
-// not enough free pages by the host count, -3: nothing to append, -4: states the pool cannot
-// take as they are).
-std::tuple<at::Tensor, at::Tensor, int64_t> pool_step_(at::Tensor handle, at::Tensor pages, at::Tensor key_states,
-                                                       at::Tensor value_states, py::buffer lens, py::buffer hw,
-                                                       int64_t free_count, bool free_exact, int64_t limit,
-                                                       int64_t flags, bool gather) {
+// A decode-step call of PagePool / QuantPagePool update or append with its host planning in C++:
+// the capacity and free-page checks of the host shadow, output allocation and the launch.  The
+// planning costs the caller about a microsecond here and 5 to 15 as array operations in Python,
+// which is what an eager step of small layers waits for.
+
+// The states of a step as the kernels take them, or false when the checked Python path must look at
+// them (it raises the exact error, or handles an empty call).
+bool step_states(const barq_kv_pool& p, const at::Tensor& pages, at::Tensor& k, at::Tensor& v) {
+  if (k.dim() != 4 || v.sizes() != k.sizes() || k.size(1) != p.kv_heads || k.size(3) != p.head_dim || !k.is_cuda() ||
+      !v.is_cuda() || k.get_device() != pages.get_device() || v.get_device() != pages.get_device() ||
+      k.scalar_type() != pages.scalar_type() || v.scalar_type() != pages.scalar_type() || k.size(0) > p.max_batch)
+    return false;
+  if (k.stride(3) != 1 || v.stride(3) != 1 || !same_layout(k, v)) {
+    k = k.contiguous();
+    v = v.contiguous();
+  }
+  return true;
+}
+
+int64_t* shadow(const py::buffer& b, int64_t batch) {
+  const py::buffer_info i = b.request(true);
+  TORCH_CHECK(i.itemsize == 8 && i.ndim == 1 && i.shape[0] >= batch && i.strides[0] == 8,
+              "a pool's host shadow is contiguous int64 arrays of at least batch entries");
+  return static_cast<int64_t*>(i.ptr);
+}
+
+struct StepPlan {
+  int64_t worst = 0;  // the longest row after the append
+  int64_t need = 0;   // pages it takes; -1: capacity exceeded, -2: not enough free pages by the host count
+};
+
+StepPlan plan_step(const barq_kv_pool& p, const int64_t* L, const int64_t* W, int64_t batch, int64_t tokens,
+                   int64_t free_count, int64_t limit) {
+  StepPlan s;
+  const int64_t P = p.page_size;
+  for (int64_t r = 0; r < batch; ++r) {
+    const int64_t end = L[r] + tokens;
+    s.worst = std::max(s.worst, end);
+    s.need += std::max<int64_t>(std::min((end + P - 1) / P, p.max_blocks) - (W[r] + P - 1) / P, 0);
+  }
+  if (s.worst > limit || s.worst > p.max_blocks * P) s.need = -1;
+  else if (s.need > free_count) s.need = -2;
+  return s;
+}
+
+void advance(int64_t* L, int64_t* W, int64_t batch, int64_t tokens) {
+  for (int64_t r = 0; r < batch; ++r) {
+    L[r] += tokens;
+    W[r] = std::max(W[r], L[r]);
+  }
+}
+
+barq_kv_pool one_pool(const at::Tensor& handle, const at::Tensor& pages) {
   TORCH_CHECK(handle.device().is_cpu() && handle.scalar_type() == at::kByte &&
                   handle.numel() == (int64_t)sizeof(barq_kv_pool),
               "not a one-pool group (see pool_group)");
   const barq_kv_pool p = *reinterpret_cast<const barq_kv_pool*>(handle.data_ptr<uint8_t>());
   TORCH_CHECK(pages.is_cuda() && pages.data_ptr() == p.key_pages, "pages do not belong to the handle");
-  at::Tensor none;
-  if (key_states.dim() != 4 || value_states.sizes() != key_states.sizes() || key_states.size(1) != p.kv_heads ||
-      key_states.size(3) != p.head_dim || !key_states.is_cuda() || !value_states.is_cuda() ||
-      key_states.get_device() != pages.get_device() || value_states.get_device() != pages.get_device() ||
-      key_states.scalar_type() != pages.scalar_type() || value_states.scalar_type() != pages.scalar_type() ||
-      key_states.size(0) > p.max_batch)
-    return {none, none, -4};
-  const int64_t batch = key_states.size(0), tokens = key_states.size(2);
-  const py::buffer_info li = lens.request(true), hi = hw.request(true);
-  TORCH_CHECK(li.itemsize == 8 && hi.itemsize == 8 && li.ndim == 1 && hi.ndim == 1 && li.shape[0] >= batch &&
-                  hi.shape[0] >= batch && li.strides[0] == 8 && hi.strides[0] == 8,
-              "lens / hw must be contiguous int64 arrays of at least batch entries");
-  int64_t* L = static_cast<int64_t*>(li.ptr);
-  int64_t* W = static_cast<int64_t*>(hi.ptr);
-  if (batch == 0 || tokens == 0) return {none, none, -3};
-  const int64_t P = p.page_size;
-  int64_t worst = 0, need = 0;
-  for (int64_t r = 0; r < batch; ++r) {
-    const int64_t end = L[r] + tokens;
-    worst = std::max(worst, end);
-    need += std::max<int64_t>(std::min((end + P - 1) / P, p.max_blocks) - (W[r] + P - 1) / P, 0);
-  }
-  if (worst > limit || worst > p.max_blocks * P) return {none, none, -1};
-  if (need > free_count) return {none, none, -2};
-  at::Tensor k = key_states, v = value_states;
-  if (k.stride(3) != 1 || v.stride(3) != 1 || !same_layout(k, v)) {
-    k = k.contiguous();
-    v = v.contiguous();
-  }
-  c10::DeviceGuard guard(pages.device());
+  return p;
+}
+
+// handle: pool_group of this one pool; pages: its key_pages (device, dtype); lens / hw: the shadow,
+// updated in place on success.  Returns (key_out, value_out, pages taken, longest row); pages taken
+// < 0 when the call must take the checked Python path instead.
+std::tuple<at::Tensor, at::Tensor, int64_t, int64_t> pool_step_(const at::Tensor& handle, const at::Tensor& pages,
+                                                                at::Tensor k, at::Tensor v, py::buffer lens,
+                                                                py::buffer hw, int64_t free_count, bool free_exact,
+                                                                int64_t limit, int64_t flags, bool gather) {
+  const barq_kv_pool p = one_pool(handle, pages);
   at::Tensor ko, vo;
+  if (!step_states(p, pages, k, v)) return {ko, vo, -4, 0};
+  const int64_t batch = k.size(0), tokens = k.size(2);
+  if (batch == 0 || tokens == 0) return {ko, vo, -3, 0};
+  int64_t* L = shadow(lens, batch);
+  int64_t* W = shadow(hw, batch);
+  const StepPlan s = plan_step(p, L, W, batch, tokens, free_count, limit);
+  if (s.need < 0) return {ko, vo, s.need, 0};
+  c10::DeviceGuard guard(pages.device());
   int rc;
   if (gather) {
-    at::Tensor both = at::empty({2, batch, p.kv_heads, worst, p.head_dim}, pages.options());
+    at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
     ko = both[0];
     vo = both[1];
     if (flags == 0 && free_exact && batch <= 64) {
@@ -446,11 +477,11 @@ std::tuple<at::Tensor, at::Tensor, int64_t> pool_step_(at::Tensor handle, at::Te
         w32[r] = (int32_t)W[r];
       }
       rc = barq_kv_update_known(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1),
-                                k.stride(2), ko.data_ptr(), vo.data_ptr(), worst, ko.stride(0), ko.stride(1),
+                                k.stride(2), ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1),
                                 ko.stride(2), l32, w32, free_count, current_stream(pages));
     } else {
       rc = barq_kv_update(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2),
-                          ko.data_ptr(), vo.data_ptr(), worst, ko.stride(0), ko.stride(1), ko.stride(2), flags,
+                          ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2), flags,
                           current_stream(pages));
     }
   } else {
@@ -458,11 +489,66 @@ std::tuple<at::Tensor, at::Tensor, int64_t> pool_step_(at::Tensor handle, at::Te
                         current_stream(pages));
   }
   check_status(rc, gather ? "pool_update_" : "pool_append_");
-  for (int64_t r = 0; r < batch; ++r) {
-    L[r] += tokens;
-    W[r] = std::max(W[r], L[r]);
+  advance(L, W, batch, tokens);
+  return {ko, vo, s.need, s.worst};
+}
+
+// A cold store packed like pool_group packs a pool.
+at::Tensor cold_group(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window) {
+  const barq_kv_pool p = pool_from(pool);
+  at::Tensor out = at::empty({(int64_t)sizeof(barq_kv_cold)}, at::kByte);
+  *reinterpret_cast<barq_kv_cold*>(out.data_ptr<uint8_t>()) = cold_from(p, pool[0], cold, window);
+  return out;
+}
+
+barq_kv_cold one_cold(const at::Tensor& handle) {
+  TORCH_CHECK(handle.device().is_cpu() && handle.scalar_type() == at::kByte &&
+                  handle.numel() == (int64_t)sizeof(barq_kv_cold),
+              "not a cold store (see cold_group)");
+  return *reinterpret_cast<const barq_kv_cold*>(handle.data_ptr<uint8_t>());
+}
+
+// pool_step_ for a pool with a cold store, of at most `chunk` tokens: also the blocks that leave the
+// window (cold_blocks: the rows' leading quantised ones, updated in place), whose compress is
+// launched only when there are any.  Returns (key_out, value_out, pages taken, longest row, blocks
+// quantised).
+std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
+    const at::Tensor& handle, const at::Tensor& cold, const at::Tensor& pages, at::Tensor k, at::Tensor v,
+    py::buffer lens, py::buffer hw, py::buffer cold_blocks, int64_t free_count, int64_t cold_free, int64_t chunk,
+    int64_t limit, int64_t flags, bool gather) {
+  const barq_kv_pool p = one_pool(handle, pages);
+  const barq_kv_cold c = one_cold(cold);
+  at::Tensor ko, vo;
+  if (!step_states(p, pages, k, v)) return {ko, vo, -4, 0, 0};
+  const int64_t batch = k.size(0), tokens = k.size(2);
+  if (batch == 0 || tokens == 0 || tokens > chunk) return {ko, vo, -3, 0, 0};
+  int64_t* L = shadow(lens, batch);
+  int64_t* W = shadow(hw, batch);
+  int64_t* C = shadow(cold_blocks, batch);
+  const StepPlan s = plan_step(p, L, W, batch, tokens, free_count, limit);
+  if (s.need < 0) return {ko, vo, s.need, 0, 0};
+  const auto frontier = [&](int64_t r) { return std::max<int64_t>(L[r] + tokens - c.window, 0) / p.page_size; };
+  int64_t moved = 0;
+  for (int64_t r = 0; r < batch; ++r) moved += std::max<int64_t>(frontier(r) - C[r], 0);
+  if (moved > cold_free) return {ko, vo, -2, 0, 0};
+  c10::DeviceGuard guard(pages.device());
+  void* stream = current_stream(pages);
+  int rc;
+  if (gather) {
+    at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
+    ko = both[0];
+    vo = both[1];
+    rc = barq_kv_update_cold(&p, &c, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2),
+                             ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2),
+                             flags | (moved == 0 ? BARQ_KV_NO_COMPRESS : 0), stream);
+  } else {
+    rc = barq_kv_append(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2), stream);
+    if (rc == BARQ_KV_OK && moved > 0) rc = barq_kv_compress(&p, &c, batch, stream);
   }
-  return {ko, vo, need};
+  check_status(rc, gather ? "pool_update_cold_" : "pool_append_");
+  for (int64_t r = 0; r < batch; ++r) C[r] = std::max(C[r], frontier(r));
+  advance(L, W, batch, tokens);
+  return {ko, vo, s.need, s.worst, moved};
 }
 
 // The pools of a model's layers packed as an array of barq_kv_pool (a CPU uint8 tensor), for
@@ -554,6 +640,48 @@ void decode_attention_into(const std::vector<at::Tensor>& pool, const barq_kv_co
   check_status(rc, "pool_decode_attention");
 }
 
+// PagePool.attend with its defaults -- an output in the query's dtype, the shadow's longest row --
+// planned here: the [batch, tokens, q_heads, head_dim] output, or an undefined tensor when the call
+// must take the checked Python path (a query the kernel does not take as it is, a workspace below
+// the launch's).
+at::Tensor pool_attend(const at::Tensor& handle, const c10::optional<at::Tensor>& cold, const at::Tensor& pages,
+                       const at::Tensor& query, py::buffer lens, double scale,
+                       const c10::optional<at::Tensor>& workspace) {
+  const barq_kv_pool p = one_pool(handle, pages);
+  const auto dt = pages.scalar_type();
+  if (!workspace.has_value() || (dt != at::kBFloat16 && dt != at::kHalf) || query.dim() != 4 || !query.is_cuda() ||
+      query.get_device() != pages.get_device() || query.scalar_type() != dt || query.size(3) != p.head_dim ||
+      query.size(1) % p.kv_heads != 0 || query.size(0) > p.max_batch || query.size(0) == 0 || query.size(2) == 0 ||
+      query.size(1) == 0 || query.stride(3) != 1 || (reinterpret_cast<uintptr_t>(query.data_ptr()) & 15) != 0 ||
+      ((query.stride(0) | query.stride(1) | query.stride(2)) & 7) != 0)
+    return at::Tensor();
+  const int64_t batch = query.size(0), heads = query.size(1), tokens = query.size(2);
+  const int64_t* L = shadow(lens, batch);
+  const int64_t max_seq = std::max<int64_t>(*std::max_element(L, L + batch), 1);
+  const at::Tensor& ws = *workspace;
+  const int64_t need = barq_kv_attention_workspace_bytes(&p, batch, heads, tokens, max_seq, 0);
+  if (need < 0 || ws.numel() < need || !ws.is_cuda() || ws.get_device() != pages.get_device() ||
+      ws.scalar_type() != at::kByte || !ws.is_contiguous())
+    return at::Tensor();
+  c10::DeviceGuard guard(pages.device());
+  at::Tensor out = at::empty({batch, tokens, heads, p.head_dim}, query.options());
+  const int64_t flags = dt == at::kHalf ? BARQ_KV_ATTN_FP16 : 0;
+  int rc;
+  if (cold.has_value()) {
+    const barq_kv_cold c = one_cold(*cold);
+    rc = barq_kv_decode_attention_cold(&p, &c, query.data_ptr(), batch, heads, tokens, query.stride(0), query.stride(1),
+                                       query.stride(2), out.data_ptr(), out.stride(0), out.stride(2), out.stride(1),
+                                       (float)scale, max_seq, 0, flags, ws.data_ptr(), ws.numel(),
+                                       current_stream(pages));
+  } else {
+    rc = barq_kv_decode_attention(&p, query.data_ptr(), batch, heads, tokens, query.stride(0), query.stride(1),
+                                  query.stride(2), out.data_ptr(), out.stride(0), out.stride(2), out.stride(1),
+                                  (float)scale, max_seq, 0, flags, ws.data_ptr(), ws.numel(), current_stream(pages));
+  }
+  check_status(rc, "pool_decode_attention");
+  return out;
+}
+
 void pool_decode_attention(std::vector<at::Tensor> pool, at::Tensor query, at::Tensor out, double scale,
                            int64_t max_seq, int64_t split_tokens, at::Tensor workspace) {
   decode_attention_into(pool, nullptr, query, out, scale, max_seq, split_tokens, workspace);
@@ -593,6 +721,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "One row selection applied to pools with cold stores, sharing quantised blocks");
   m.def("pool_group", &pool_group, "Pack the pools of a model's layers for the batched entry points");
   m.def("pool_step_", &pool_step_, "One update / append with its host planning (see PagePool.update)");
+  m.def("cold_group", &cold_group, "Pack a pool's cold store for pool_step_cold_ and pool_attend");
+  m.def("pool_step_cold_", &pool_step_cold_, "pool_step_ for a pool with a cold store (see QuantPagePool.update)");
+  m.def("pool_attend", &pool_attend, "Decode attention with its host planning (see PagePool.attend)");
   m.def("select_workspace_words", &select_workspace_words, "Workspace words of pool_group_select_rows_");
   m.def("pool_group_select_rows_", &pool_group_select_rows_,
         "One row selection applied to every pool of a group, sharing full pages");

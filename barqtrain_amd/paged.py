@@ -55,10 +55,16 @@ class PagedKVPoolExhausted(PagedKVCapacityError):
     """The pool has fewer free pages than an append needs."""
 
 
-def _gpu_backend():
-    from barqtrain_amd import kv_cache
+_KV_CACHE = None  # the kv_cache module, which imports this one
 
-    backend = kv_cache._get_cuda_backend()
+
+def _gpu_backend():
+    global _KV_CACHE
+    if _KV_CACHE is None:
+        from barqtrain_amd import kv_cache
+
+        _KV_CACHE = kv_cache
+    backend = _KV_CACHE._get_cuda_backend()
     if backend is None or not hasattr(backend, "pool_update_"):
         raise RuntimeError(
             "barqtrain: the HIP backend module barqtrain_cuda is not available; build it with "
@@ -115,7 +121,13 @@ class PagePool:
         self.shared = False      # some page may be held by more than one block
         self.tails_shared = False  # a crop may have left shared pages in rows' tails
         self.generation = 0      # bumped whenever the tensors are replaced (cached pool groups)
+        self._handle = None      # the tensors packed for the binding, of one generation
+        self._attn_ws = None     # decode attention's workspace
         self.reset(page_order)
+
+    def __getstate__(self):
+        # A copy packs its own tensors and takes its own workspace.
+        return {**self.__dict__, "_handle": None, "_attn_ws": None}
 
     # ------------------------------------------------------------------ plumbing
     @property
@@ -241,18 +253,32 @@ class PagePool:
     def _step(self, key_states, value_states, max_length, flags, gather):
         """One update (gather) or append with the host planning done in the binding (pool_step_):
         returns (key_out, value_out, pages taken), or pages taken < 0 when the call must take the
-        checked path (which raises the exact error, or handles an empty call)."""
+        checked path (which raises the exact error, or handles an empty call), and the longest row
+        after the call."""
         backend = _gpu_backend()
-        handle = self.__dict__.get("_handle")
-        if handle is None or handle[0] != self.generation:
-            handle = (self.generation, backend.pool_group([self.tensors]))
-            self._handle = handle
         limit = self.capacity if max_length is None else int(max_length)
-        ko, vo, need = backend.pool_step_(handle[1], self.key_pages, key_states, value_states, self.lens, self.hw,
-                                          self.free_count, self.free_exact, limit, flags, gather)
+        ko, vo, need, worst = backend.pool_step_(self._packed(backend)[1], self.key_pages, key_states, value_states,
+                                                 self.lens, self.hw, self.free_count, self.free_exact, limit, flags,
+                                                 gather)
         if need >= 0:
             self.free_count -= need
-        return ko, vo, need
+        return ko, vo, need, worst
+
+    def _packed(self, backend):
+        """(generation, pool, cold store or None): the pool's tensors packed for the binding's step
+        calls, packed again when they are replaced."""
+        handle = self._handle
+        if handle is None or handle[0] != self.generation:
+            handle = self._handle = (self.generation, backend.pool_group([self.tensors]), None)
+        return handle
+
+    def step(self, key_states: torch.Tensor, value_states: torch.Tensor, max_length: int, gather: bool):
+        """An eager decode step: ``(K, V, longest row)`` of an update (K and V None for an append),
+        or None, nothing changed, when `update` / `append` have to look at the call."""
+        if self.device.type != "cuda":
+            return None
+        ko, vo, need, worst = self._step(key_states, value_states, max_length, 0, gather)
+        return (ko, vo, worst) if need >= 0 else None
 
     def append(self, key_states: torch.Tensor, value_states: torch.Tensor,
                max_length: Optional[int] = None) -> None:
@@ -326,7 +352,7 @@ class PagePool:
                flags: int = 0) -> tuple[torch.Tensor, torch.Tensor]:
         """Append, then materialise rows [0, batch) up to the longest row, in one pass."""
         if self.on_gpu and out is None and seq_out is None:
-            ko, vo, need = self._step(key_states, value_states, max_length, flags, True)
+            ko, vo, need, _ = self._step(key_states, value_states, max_length, flags, True)
             if need >= 0:
                 return ko, vo
         self._check_states(key_states, value_states)
@@ -472,6 +498,10 @@ class PagePool:
         ``[batch, tokens, q_heads, head_dim]`` buffer, the layout attention outputs take next)
         in `out_dtype` (default the query's).  `max_seq` bounds the rows' lengths (default:
         the host shadow's longest row; pass the capacity when capturing a graph)."""
+        if out is None and out_dtype is None and split_tokens == 0 and max_seq is None:
+            got = self._attend_step(query, scale)
+            if got is not None:
+                return got.transpose(1, 2)
         if query.dim() != 4 or query.shape[3] != self.head_dim or query.shape[1] % self.kv_heads:
             raise ValueError("query must be [batch, q_heads, tokens, head_dim] with q_heads a "
                              "multiple of the pool's kv_heads")
@@ -507,13 +537,23 @@ class PagePool:
                              self.attention_workspace(need))
         return out
 
+    def _attend_step(self, query: torch.Tensor, scale: Optional[float]) -> Optional[torch.Tensor]:
+        """attend with its defaults, planned in the binding: ``[batch, tokens, q_heads, head_dim]``,
+        or None when `attend` has to look at the call (or to allocate the workspace)."""
+        if self.device.type != "cuda" or self._attn_ws is None:
+            return None
+        backend = _gpu_backend()
+        scale = 1.0 / math.sqrt(self.head_dim) if scale is None else float(scale)
+        handle = self._packed(backend)
+        return backend.pool_attend(handle[1], handle[2], self.key_pages, query, self.lens, scale, self._attn_ws)
+
     def _attention_call(self, backend, query, out, scale, max_seq, split_tokens, ws):
         backend.pool_decode_attention(self.tensors, query, out, scale, max_seq, split_tokens, ws)
 
     def attention_workspace(self, nbytes: int) -> torch.Tensor:
         """The pool's decode-attention workspace (split records), at least `nbytes`; grown, never
         shrunk.  Launches on one stream may share it."""
-        ws = getattr(self, "_attn_ws", None)
+        ws = self._attn_ws
         if ws is None or ws.numel() < nbytes:
             ws = torch.empty((max(int(nbytes), 256),), dtype=torch.uint8, device=self.device)
             self._attn_ws = ws
@@ -636,8 +676,34 @@ class QuantPagePool(PagePool):
         self.cold_free -= moved
         self.free_count += moved  # each quantised block returned its full-precision page
 
+    def _packed(self, backend):
+        handle = self._handle
+        if handle is None or handle[0] != self.generation:
+            handle = self._handle = (self.generation, backend.pool_group([self.tensors]),
+                                     backend.cold_group(self.tensors, self.cold_tensors, self.window))
+        return handle
+
+    def _step(self, key_states, value_states, max_length, flags, gather):
+        backend = _gpu_backend()
+        handle = self._packed(backend)
+        limit = self.capacity if max_length is None else int(max_length)
+        ko, vo, need, worst, moved = backend.pool_step_cold_(
+            handle[1], handle[2], self.key_pages, key_states, value_states, self.lens, self.hw, self.cold_blocks,
+            self.free_count, self.cold_free, self.chunk, limit, flags, gather)
+        if need >= 0:
+            self.free_count += moved - need  # each quantised block returned its full-precision page
+            self.cold_free -= moved
+        return ko, vo, need, worst
+
+    def _attend_step(self, query, scale):
+        if self.page_size % 16 or self.head_dim not in (64, 128):  # attends over its gather
+            return None
+        return super()._attend_step(query, scale)
+
     def append(self, key_states: torch.Tensor, value_states: torch.Tensor,
                max_length: Optional[int] = None) -> None:
+        if self.on_gpu and self._step(key_states, value_states, max_length, 0, False)[2] >= 0:
+            return
         self._check_states(key_states, value_states)
         batch, _, tokens, _ = key_states.shape
         if tokens > self.chunk:
@@ -754,6 +820,10 @@ class QuantPagePool(PagePool):
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor,
                max_length: Optional[int] = None, out=None, seq_out: Optional[int] = None,
                flags: int = 0) -> tuple[torch.Tensor, torch.Tensor]:
+        if self.on_gpu and out is None and seq_out is None:
+            ko, vo, need, _ = self._step(key_states, value_states, max_length, flags, True)
+            if need >= 0:
+                return ko, vo
         self._check_states(key_states, value_states)
         batch, _, tokens, _ = key_states.shape
         if tokens > self.chunk:
