@@ -89,8 +89,9 @@ constexpr int64_t kLongChunksPerPart = 72;
 
 enum : int { kBF16 = 0, kF16 = 1 };
 
-// Head sizes the kernels are built for (HD = 64, 128, and 256 on two-byte pages through the flat
-// schedule at one wave per SIMD) and the lane layout each gives.  Scores:
+// Head sizes the kernels are built for (HD = 64, 128, and 256 on two-byte pages: the pair kernel
+// for up to 4 query rows, else the flat schedule at one wave per SIMD) and the lane layout each
+// gives.  Scores:
 // lane (g, n16) of the 16x16x32 MFMA holds dims 32 * step + 8 * g .. +7 of one position, HD / 32
 // steps.  V: a position's HD dims are HD / 8 lanes of 8 dims, so one 16-byte load per lane covers
 // 64 / (HD / 8) positions and a chunk takes 16 / that many loads.
@@ -469,7 +470,8 @@ __device__ __forceinline__ void load_chunk(const AttnArgs& a, const int (&pt)[kT
 // A chunk of a two-byte pool with whole-chunk pages whose positions past `end` read position
 // end - 1 (the causal mask gives them probability 0): every lane loads, no branch around the loads.
 // QORDER: K in the quantised pools' order (issue_query), for the two-byte pages of such a pool.
-template <int HD, bool QORDER = false>
+// K, V: which of the two.
+template <int HD, bool QORDER = false, bool K = true, bool V = true>
 __device__ __forceinline__ void load_chunk_clamped(const AttnArgs& a, const int (&pt)[kTableRegs], int blk0,
                                                    const char* kbase, const char* vbase, int tc, int end, int n16,
                                                    int g, int vpos, int vdim, u32x4 (&kv)[Head<HD>::kSteps],
@@ -484,12 +486,16 @@ __device__ __forceinline__ void load_chunk_clamped(const AttnArgs& a, const int 
   const int64_t base =
       (int64_t)page * a.page_bytes + (int64_t)(tc - (int)(blk * (uint32_t)a.page_size)) * a.row_bytes;
   const int lastp = end - 1 - tc;  // >= 15 for a whole chunk
-  const char* kp = kbase + base + min(n16, lastp) * a.row_bytes + (QORDER ? 16 * kSteps * g : 16 * g);
+  if constexpr (K) {
+    const char* kp = kbase + base + min(n16, lastp) * a.row_bytes + (QORDER ? 16 * kSteps * g : 16 * g);
 #pragma unroll
-  for (int st = 0; st < kSteps; ++st) kv[st] = ld_page_k(kp + (QORDER ? 16 : 64) * st);
+    for (int st = 0; st < kSteps; ++st) kv[st] = ld_page_k(kp + (QORDER ? 16 : 64) * st);
+  }
+  if constexpr (V) {
 #pragma unroll
-  for (int s = 0; s < kVLoads; ++s)
-    vv[s] = ld_page(vbase + base + min(kVPos * s + vpos, lastp) * a.row_bytes + 16 * vdim);
+    for (int s = 0; s < kVLoads; ++s)
+      vv[s] = ld_page(vbase + base + min(kVPos * s + vpos, lastp) * a.row_bytes + 16 * vdim);
+  }
 }
 
 // A quantised chunk (its block's table entry is -2 - c, c its quantised block), positions past
@@ -672,7 +678,7 @@ __device__ void attend_piece(const AttnArgs& a, float (&lp)[kBlock][kMaxRows],
   int pt[kTableRegs];
   // The pair kernel keeps its query fragments in registers (it has them to spare), the others
   // read them from LDS for every chunk.
-  constexpr bool kQReg = PRE && !COLD && R == 1;
+  constexpr bool kQReg = PRE && !COLD && R == 1 && HD <= 128;
   u32x4 qreg[kSteps];
   {
     u32x4 qv[kSteps];
@@ -737,7 +743,7 @@ __device__ void attend_piece(const AttnArgs& a, float (&lp)[kBlock][kMaxRows],
   // (with the rescale under a branch, the quantised flat kernel and 8+ rows on the flat schedule
   // or over quantised pages spill)
   constexpr bool kLazyMax = R == 1 ? !COLD || PRE : R == 2 && PRE && !COLD;
-  auto compute = [&](int tc, const u32x4 (&kv)[kSteps], u32x4 (&vv)[kVLoads], bool kcodes, bool vcold) {
+  auto score = [&](int tc, const u32x4 (&kv)[kSteps], bool kcodes) {
     // Scores: lane (g, n16), register r = row 4g + r, position tc + n16; log2 units.
     f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -811,6 +817,8 @@ __device__ void attend_piece(const AttnArgs& a, float (&lp)[kBlock][kMaxRows],
           for (int e = 0; e < 8; ++e) acc[r2][e][m] *= al;
         }
     }
+  };
+  auto weigh = [&](u32x4 (&vv)[kVLoads], bool vcold) {
     bool vcodes = false;
     if (COLD && vcold) {
       vcodes = __builtin_amdgcn_ballot_w64(!scales_moderate<true>(vv)) == 0;
@@ -837,6 +845,10 @@ __device__ void attend_piece(const AttnArgs& a, float (&lp)[kBlock][kMaxRows],
       }
     }
   };
+  auto compute = [&](int tc, const u32x4 (&kv)[kSteps], u32x4 (&vv)[kVLoads], bool kcodes, bool vcold) {
+    score(tc, kv, kcodes);
+    weigh(vv, vcold);
+  };
 
   // Two register buffers: the next chunk's loads are in flight while one is computed (a third
   // spills, or for 4 query rows runs slower, with the accumulators in registers).
@@ -852,7 +864,34 @@ __device__ void attend_piece(const AttnArgs& a, float (&lp)[kBlock][kMaxRows],
     compute(tc, kr[i], vr[i], kcodes, COLD && cr[i]);
     tc += kBlock;
   };
-  if constexpr (PRE && !COLD && R == 1) {
+  if constexpr (PRE && !COLD && HD == 256) {
+    // A 256-dim chunk is 128 registers of K and V over two buffers: with the accumulators that left
+    // one wave per SIMD.  One buffer each, loaded again as soon as it is used up -- the next chunk's
+    // K while this one's V is weighed, its V while the next scores are made -- keeps a chunk (16
+    // KiB) a wave in flight at two waves per SIMD.  Loads on every path, as below.
+    auto load_k = [&](int t) {
+      load_chunk_clamped<HD, false, true, false>(a, pt, blk0, kbase, vbase, t, t_end, n16, g, vpos, vdim, kr[0], vr[0]);
+    };
+    auto load_v = [&](int t) {
+      load_chunk_clamped<HD, false, false, true>(a, pt, blk0, kbase, vbase, t, t_end, n16, g, vpos, vdim, kr[0], vr[0]);
+    };
+    if (tc < t_end) {
+      load_k(tc);
+      load_v(tc);
+      for (;;) {
+        score(tc, kr[0], false);
+        __builtin_amdgcn_sched_barrier(0);
+        if (tc + kBlock >= t_end) break;
+        load_k(tc + kBlock);
+        __builtin_amdgcn_sched_barrier(0);
+        weigh(vr[0], false);
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(tc + kBlock);
+        tc += kBlock;
+      }
+      weigh(vr[0], false);
+    }
+  } else if constexpr (PRE && !COLD && R == 1) {
     // Pair kernel, up to 4 query rows, two-byte pages (its table window holds every block of the
     // pair: no slide).  The wait the compiler puts before a chunk's products counts the loads
     // issued after that chunk's; where one path to the products skips the next chunk's loads, or
@@ -1369,8 +1408,11 @@ int resident_waves(K kernel) {
 template <int HD, int E, int R, bool U, typename OutT, bool COLD>
 hipError_t launch_typed(AttnArgs a, bool merge, hipStream_t stream) {
   // Pairs of bounded length, the automatic split, whole-chunk pages, up to 8 query rows (two waves
-  // per SIMD keep the accumulators in registers): one workgroup per pair.
-  if constexpr (U && R <= 2 && HD <= 128) {
+  // per SIMD keep the accumulators in registers): one workgroup per pair.  Head size 256: up to 4
+  // rows (12 rows x 4 heads x 1500 positions, G 2, T 2: 28.0 -> 19.2 us against the flat pair of
+  // launches; 64 x 4 x 650: 41.5 -> 31.4; 64 x 4 x 1900: 102 -> 88).  With 5 to 8 its accumulators
+  // spill and it lost from ~300 positions on (1 x 3000: 20.2 -> 28.8; 16 x 4 x 700: 25.0 -> 27.0).
+  if constexpr (U && R <= 2 && (HD <= 128 || (R == 1 && !COLD))) {
     const int64_t pairs = (int64_t)a.batch * a.kv_heads;
     // Fewer pairs than kPairMinPairs leave CUs idle, but up to kPairMaxChunks a pair one launch
     // still beats the flat pair of launches and its merge (C2 shape at batch 1: 650 positions
@@ -1404,13 +1446,16 @@ hipError_t launch_typed(AttnArgs a, bool merge, hipStream_t stream) {
     }
     // Longer rows at small batches (C4 at 32k positions: 34.3 -> 31.1 us against the flat pair of
     // launches): up to kMaxSplitLong workgroups a pair, each part's blocks in a window of its own.
-    if (a.range_chunks == 0 && pairs > 0 && pairs <= BARQ_KV_CTRL_PAIR_SLOTS) {
-      auto* split_long = attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitLong>;
-      const int64_t nlong =
-          std::min<int64_t>(kMaxSplitLong, resident_blocks<kPairWaves * kWave>(split_long, 0) / pairs);
-      if (nlong > 2 && chunks <= nlong * kLongChunksPerPart) {
-        hipLaunchKernelGGL(split_long, dim3((unsigned)(nlong * pairs)), dim3(kPairWaves * kWave), 0, stream, a);
-        return hipGetLastError();
+    // (Head size 256 keeps the flat schedule there: 1 x 30000 positions, G 4: 24.2 against 31.8 us.)
+    if constexpr (HD <= 128) {
+      if (a.range_chunks == 0 && pairs > 0 && pairs <= BARQ_KV_CTRL_PAIR_SLOTS) {
+        auto* split_long = attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitLong>;
+        const int64_t nlong =
+            std::min<int64_t>(kMaxSplitLong, resident_blocks<kPairWaves * kWave>(split_long, 0) / pairs);
+        if (nlong > 2 && chunks <= nlong * kLongChunksPerPart) {
+          hipLaunchKernelGGL(split_long, dim3((unsigned)(nlong * pairs)), dim3(kPairWaves * kWave), 0, stream, a);
+          return hipGetLastError();
+        }
       }
     }
   }
