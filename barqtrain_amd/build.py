@@ -26,7 +26,7 @@ LIB_NAME = "libbarq_kv.so"
 EXT_NAME = "barqtrain_cuda"
 OFFLOAD_ARCH = "gfx950"
 HIP_SOURCES = ("barq_kv.hip", "barq_kv_attention.hip", "barq_kv_quant.hip")
-HIP_HEADERS = ("fastdiv.h", "barq_kv_fp8.h", "barq_kv_commit.h")
+HIP_HEADERS = ("fastdiv.h", "barq_kv_fp8.h", "barq_kv_commit.h", "barq_kv_internal.h")
 HOST_SOURCES = ("barq_kv_torch.cpp",)
 
 
@@ -124,7 +124,7 @@ def _extension_commands(obj: Path, tmp: Path) -> tuple[list[str], list[str]]:
         f"-DTORCH_EXTENSION_NAME={EXT_NAME}", "-DTORCH_API_INCLUDE_EXTENSION_H",
         f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
         *[f"-I{p}" for p in cpp_extension.include_paths(device_type="cuda")],
-        f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}",
+        f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}", f"-I{INCLUDE}", f"-I{CSRC}",
         *(str(CSRC / f) for f in HOST_SOURCES), "-o", str(obj),
     ]
     link_cmd = [

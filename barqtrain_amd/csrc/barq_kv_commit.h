@@ -80,8 +80,10 @@ __device__ __forceinline__ NewBlocks new_blocks(int len, int hw, int tokens, int
 // holds row r's length and high-water mark, lane k holds free_pages[top - 1 - k], the page the
 // k-th new block takes.  The new blocks are mapped one rank per lane, 64 ranks a round; ranks
 // past the first 64 read their page from the stack, eight rounds' reads in flight at once.
+// MAPPED: lane r's row is row_of instead of r.
+template <bool MAPPED = false>
 __device__ inline void commit_from_lanes(const barq_kv_pool& p, int batch, int tokens, int limit,
-                                  const FastDiv& div_page, int len, int hw, int top, int free_k) {
+                                  const FastDiv& div_page, int len, int hw, int top, int free_k, int row_of = 0) {
   const int lane = threadIdx.x & (kWave - 1);
   const int mb = (int)p.max_blocks;
   int err = 0;
@@ -114,6 +116,7 @@ __device__ inline void commit_from_lanes(const barq_kv_pool& p, int batch, int t
       const int src = row & (kWave - 1);
       const int row_first = __shfl(nb.first, src, kWave);
       const int row_excl = __shfl(incl - nb.count, src, kWave);
+      if constexpr (MAPPED) row = __shfl(row_of, src, kWave);
       if (k < total) {
         const int page = top - 1 - k >= 0 ? checked_page(pg[u], p.num_pages) : -1;
         if (page < 0) err |= BARQ_KV_ERRBIT_POOL_EXHAUSTED;
@@ -122,8 +125,9 @@ __device__ inline void commit_from_lanes(const barq_kv_pool& p, int batch, int t
     }
   }
   if (lane < batch) {
-    p.seq_lens[lane] = len + tokens;
-    p.high_water[lane] = max(hw, len + tokens);
+    const int r = MAPPED ? row_of : lane;
+    p.seq_lens[r] = len + tokens;
+    p.high_water[r] = max(hw, len + tokens);
   }
   if (lane == 0) p.ctrl[BARQ_KV_CTRL_FREE_TOP] = max(0, top - total);
   if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);

@@ -1,0 +1,19 @@
+// Between libbarq_kv.so and its torch binding, beside the C ABI of include/barq_kv.h: calls that only a
+// caller with the binding's host shadow makes.  Not part of the ABI.
+
+#pragma once
+
+#include <stdint.h>
+
+#include "barq_kv.h"
+
+namespace barq_internal {
+
+// barq_kv_append of key_states[i] to row rows[i] (rows null: row i), i < batch <= 64, for a caller
+// that knows the rows' lengths and marks and the free stack's top exactly.  BARQ_KV_ERR_UNSUPPORTED,
+// nothing launched, for more rows or states and pools that 16-byte vectors do not fit.
+int append_known(const barq_kv_pool* pool, const void* key_states, const void* value_states, int64_t batch,
+                 int64_t tokens, int64_t stride_b, int64_t stride_h, int64_t stride_t, const int32_t* rows,
+                 const int32_t* seq_lens, const int32_t* high_water, int64_t free_top, void* stream);
+
+}  // namespace barq_internal

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "barq_kv.h"
+#include "barq_kv_internal.h"
 
 namespace {
 
@@ -438,6 +439,26 @@ void advance(int64_t* L, int64_t* W, int64_t batch, int64_t tokens) {
   }
 }
 
+// An append from the shadow's state where it is exact, else from the device's.
+int append_step(const barq_kv_pool& p, const at::Tensor& k, const at::Tensor& v, const int64_t* L, const int64_t* W,
+                const int64_t* rows, int64_t free_count, bool free_exact, void* stream) {
+  const int64_t batch = k.size(0), tokens = k.size(2);
+  if (free_exact && batch <= 64) {
+    int32_t l32[64], w32[64], r32[64];
+    for (int64_t i = 0; i < batch; ++i) {
+      const int64_t r = rows ? rows[i] : i;
+      l32[i] = (int32_t)L[r];
+      w32[i] = (int32_t)W[r];
+      r32[i] = (int32_t)r;
+    }
+    const int rc = barq_internal::append_known(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1),
+                                               k.stride(2), r32, l32, w32, free_count, stream);
+    if (rc != BARQ_KV_ERR_UNSUPPORTED) return rc;
+  }
+  if (rows) return BARQ_KV_ERR_UNSUPPORTED;
+  return barq_kv_append(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2), stream);
+}
+
 barq_kv_pool one_pool(const at::Tensor& handle, const at::Tensor& pages) {
   TORCH_CHECK(handle.device().is_cpu() && handle.scalar_type() == at::kByte &&
                   handle.numel() == (int64_t)sizeof(barq_kv_pool),
@@ -485,12 +506,28 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t> pool_step_(const at::Tensor
                           current_stream(pages));
     }
   } else {
-    rc = barq_kv_append(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2),
-                        current_stream(pages));
+    rc = append_step(p, k, v, L, W, nullptr, free_count, free_exact, current_stream(pages));
   }
   check_status(rc, gather ? "pool_update_" : "pool_append_");
   advance(L, W, batch, tokens);
   return {ko, vo, s.need, s.worst};
+}
+
+// k[i], v[i] appended to row rows[i] in one launch, from the shadow's exact state (checked by the caller;
+// the shadow is not advanced); false, nothing launched, when the kernel does not take the call.
+bool pool_append_rows_(const at::Tensor& handle, const at::Tensor& pages, at::Tensor k, at::Tensor v,
+                       const std::vector<int64_t>& rows, py::buffer lens, py::buffer hw, int64_t free_count) {
+  const barq_kv_pool p = one_pool(handle, pages);
+  if (!step_states(p, pages, k, v) || (int64_t)rows.size() != k.size(0) || k.size(0) > 64) return false;
+  const int64_t* L = shadow(lens, p.max_batch);
+  const int64_t* W = shadow(hw, p.max_batch);
+  for (const int64_t r : rows)
+    if (r < 0 || r >= p.max_batch) return false;
+  c10::DeviceGuard guard(pages.device());
+  const int rc = append_step(p, k, v, L, W, rows.data(), free_count, true, current_stream(pages));
+  if (rc == BARQ_KV_ERR_UNSUPPORTED) return false;
+  check_status(rc, "pool_append_rows_");
+  return true;
 }
 
 // A cold store packed like pool_group packs a pool.
@@ -514,8 +551,8 @@ barq_kv_cold one_cold(const at::Tensor& handle) {
 // quantised).
 std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
     const at::Tensor& handle, const at::Tensor& cold, const at::Tensor& pages, at::Tensor k, at::Tensor v,
-    py::buffer lens, py::buffer hw, py::buffer cold_blocks, int64_t free_count, int64_t cold_free, int64_t chunk,
-    int64_t limit, int64_t flags, bool gather) {
+    py::buffer lens, py::buffer hw, py::buffer cold_blocks, int64_t free_count, bool free_exact, int64_t cold_free,
+    int64_t chunk, int64_t limit, int64_t flags, bool gather) {
   const barq_kv_pool p = one_pool(handle, pages);
   const barq_kv_cold c = one_cold(cold);
   at::Tensor ko, vo;
@@ -542,7 +579,7 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
                              ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2),
                              flags | (moved == 0 ? BARQ_KV_NO_COMPRESS : 0), stream);
   } else {
-    rc = barq_kv_append(&p, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2), stream);
+    rc = append_step(p, k, v, L, W, nullptr, free_count, free_exact, stream);
     if (rc == BARQ_KV_OK && moved > 0) rc = barq_kv_compress(&p, &c, batch, stream);
   }
   check_status(rc, gather ? "pool_update_cold_" : "pool_append_");
@@ -721,6 +758,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "One row selection applied to pools with cold stores, sharing quantised blocks");
   m.def("pool_group", &pool_group, "Pack the pools of a model's layers for the batched entry points");
   m.def("pool_step_", &pool_step_, "One update / append with its host planning (see PagePool.update)");
+  m.def("pool_append_rows_", &pool_append_rows_, "Append to any rows in one launch (see PagePool.append_rows)");
   m.def("cold_group", &cold_group, "Pack a pool's cold store for pool_step_cold_ and pool_attend");
   m.def("pool_step_cold_", &pool_step_cold_, "pool_step_ for a pool with a cold store (see QuantPagePool.update)");
   m.def("pool_attend", &pool_attend, "Decode attention with its host planning (see PagePool.attend)");

@@ -297,9 +297,9 @@ class PagePool:
                     max_length: Optional[int] = None) -> None:
         """Append ``key_states[i]`` / ``value_states[i]`` to row ``rows[i]`` (distinct rows, not
         necessarily [0, batch)): a freed row takes a new sequence's prefill while the others keep
-        decoding.  Checked in full first (capacity, free pages), then one append launch per row
-        over the one-row view of the row metadata -- the same kernels, sharing the free stack,
-        so pages come off it in the order of `rows`."""
+        decoding.  Checked in full first (capacity, free pages), then one append launch for up to
+        64 rows whose state the host knows exactly, else one per row over the one-row view of the
+        row metadata.  Pages come off the stack in the order of `rows` either way."""
         self._check_states(key_states, value_states)
         rows = [int(r) for r in rows]
         if len(rows) != key_states.shape[0]:
@@ -322,9 +322,11 @@ class PagePool:
         k, v = self._compatible_pair(key_states, value_states)
         t = self.tensors
         ops = self._ops()
-        for i, row in enumerate(rows):
-            one = t[:2] + [t[2][row:row + 1], t[3][row:row + 1], t[4][row:row + 1]] + t[5:]
-            ops.pool_append_(one, k[i:i + 1], v[i:i + 1])
+        if not (self.on_gpu and self.free_exact and ops.pool_append_rows_(
+                self._packed(ops)[1], self.key_pages, k, v, rows, self.lens, self.hw, self.free_count)):
+            for i, row in enumerate(rows):
+                one = t[:2] + [t[2][row:row + 1], t[3][row:row + 1], t[4][row:row + 1]] + t[5:]
+                ops.pool_append_(one, k[i:i + 1], v[i:i + 1])
         self.lens[r] += tokens
         self.hw[r] = np.maximum(self.hw[r], self.lens[r])
         self.free_count -= need
@@ -689,7 +691,7 @@ class QuantPagePool(PagePool):
         limit = self.capacity if max_length is None else int(max_length)
         ko, vo, need, worst, moved = backend.pool_step_cold_(
             handle[1], handle[2], self.key_pages, key_states, value_states, self.lens, self.hw, self.cold_blocks,
-            self.free_count, self.cold_free, self.chunk, limit, flags, gather)
+            self.free_count, self.free_exact, self.cold_free, self.chunk, limit, flags, gather)
         if need >= 0:
             self.free_count += moved - need  # each quantised block returned its full-precision page
             self.cold_free -= moved
