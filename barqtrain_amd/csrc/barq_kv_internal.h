@@ -16,4 +16,11 @@ int append_known(const barq_kv_pool* pool, const void* key_states, const void* v
                  int64_t tokens, int64_t stride_b, int64_t stride_h, int64_t stride_t, const int32_t* rows,
                  const int32_t* seq_lens, const int32_t* high_water, int64_t free_top, void* stream);
 
+// barq_kv_crop of rows [0, batch) of n pools, whose row lengths are at seq_lens[i].
+int crop_layers(int32_t* const* seq_lens, int64_t n, int64_t batch, int64_t max_length, void* stream);
+
+// barq_kv_pool_reset (no page order) of n pools, with colds (one per pool, or null) also
+// barq_kv_cold_reset.
+int reset_layers(const barq_kv_pool* pools, const barq_kv_cold* colds, int64_t n, void* stream);
+
 }  // namespace barq_internal

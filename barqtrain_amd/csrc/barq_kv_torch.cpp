@@ -545,6 +545,56 @@ barq_kv_cold one_cold(const at::Tensor& handle) {
   return *reinterpret_cast<const barq_kv_cold*>(handle.data_ptr<uint8_t>());
 }
 
+// A crop of rows [0, batch) of a model's layers in one launch: the pools' row lengths, their host
+// shadows (updated in place) and, for pools with cold stores, the rows' leading quantised blocks.
+// False, nothing done, when a crop would re-open a quantised block (colds[i][r] * page_sizes[i] past
+// the row's new length).
+bool crop_layers_(const std::vector<at::Tensor>& seq_lens, const std::vector<py::buffer>& lens,
+                  const std::vector<c10::optional<py::buffer>>& colds, const std::vector<int64_t>& page_sizes,
+                  int64_t batch, int64_t max_length) {
+  const size_t n = seq_lens.size();
+  TORCH_CHECK(n > 0 && lens.size() == n && colds.size() == n && page_sizes.size() == n && max_length >= 0,
+              "crop_layers_: one entry per pool");
+  std::vector<int32_t*> device(n);
+  std::vector<int64_t*> host(n);
+  for (size_t i = 0; i < n; ++i) {
+    const at::Tensor& t = seq_lens[i];
+    TORCH_CHECK(t.is_cuda() && t.get_device() == seq_lens[0].get_device() && t.scalar_type() == at::kInt &&
+                    t.is_contiguous() && t.numel() >= batch,
+                "row lengths must be contiguous int32 on one device");
+    device[i] = t.data_ptr<int32_t>();
+    host[i] = shadow(lens[i], batch);
+    if (colds[i].has_value()) {
+      const int64_t* c = shadow(*colds[i], batch);
+      for (int64_t r = 0; r < batch; ++r)
+        if (c[r] > std::min(host[i][r], max_length) / page_sizes[i]) return false;
+    }
+  }
+  c10::DeviceGuard guard(seq_lens[0].device());
+  check_status(barq_internal::crop_layers(device.data(), (int64_t)n, batch, max_length, current_stream(seq_lens[0])),
+               "crop_layers_");
+  for (int64_t* L : host)
+    for (int64_t r = 0; r < batch; ++r) L[r] = std::min(L[r], max_length);
+  return true;
+}
+
+// Reset of a model's pools, packed by pool_group and (all of them or none) cold_group, in one launch; like: a tensor of theirs (device, stream).
+void reset_layers_(const std::vector<at::Tensor>& pools, const std::vector<at::Tensor>& colds, const at::Tensor& like) {
+  TORCH_CHECK(like.is_cuda() && (colds.empty() || colds.size() == pools.size()), "reset_layers_: one cold store per pool");
+  std::vector<barq_kv_pool> ps;
+  std::vector<barq_kv_cold> cs;
+  for (const at::Tensor& t : pools) {
+    TORCH_CHECK(t.device().is_cpu() && t.scalar_type() == at::kByte && t.numel() == (int64_t)sizeof(barq_kv_pool),
+                "not a one-pool group (see pool_group)");
+    ps.push_back(*reinterpret_cast<const barq_kv_pool*>(t.data_ptr<uint8_t>()));
+  }
+  for (const at::Tensor& t : colds) cs.push_back(one_cold(t));
+  c10::DeviceGuard guard(like.device());
+  check_status(barq_internal::reset_layers(ps.data(), cs.empty() ? nullptr : cs.data(), (int64_t)ps.size(),
+                                           current_stream(like)),
+               "reset_layers_");
+}
+
 // pool_step_ for a pool with a cold store, of at most `chunk` tokens: also the blocks that leave the
 // window (cold_blocks: the rows' leading quantised ones, updated in place), whose compress is
 // launched only when there are any.  Returns (key_out, value_out, pages taken, longest row, blocks
@@ -759,6 +809,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pool_group", &pool_group, "Pack the pools of a model's layers for the batched entry points");
   m.def("pool_step_", &pool_step_, "One update / append with its host planning (see PagePool.update)");
   m.def("pool_append_rows_", &pool_append_rows_, "Append to any rows in one launch (see PagePool.append_rows)");
+  m.def("crop_layers_", &crop_layers_, "Crop of a model's layers in one launch (see paged.crop_layers)");
+  m.def("reset_layers_", &reset_layers_, "Reset of a model's layers in one launch (see paged.reset_layers)");
   m.def("cold_group", &cold_group, "Pack a pool's cold store for pool_step_cold_ and pool_attend");
   m.def("pool_step_cold_", &pool_step_cold_, "pool_step_ for a pool with a cold store (see QuantPagePool.update)");
   m.def("pool_attend", &pool_attend, "Decode attention with its host planning (see PagePool.attend)");

@@ -227,6 +227,10 @@ class PagePool:
                     torch.arange(self.num_pages, dtype=torch.int32, device=self.device)):
                 raise ValueError("page_order must list every page of the pool exactly once")
         self._ops().pool_reset_(self.tensors, page_order)
+        self._emptied()
+
+    def _emptied(self) -> None:
+        """The host's shadow of an empty pool."""
         self.lens[:] = 0
         self.hw[:] = 0
         self.free_count = self.num_pages
@@ -651,6 +655,9 @@ class QuantPagePool(PagePool):
     def reset(self, page_order: Optional[torch.Tensor] = None) -> None:
         super().reset(page_order)
         self._ops().pool_cold_reset_(self.tensors, self.cold_tensors, self.window)
+
+    def _emptied(self) -> None:
+        super()._emptied()
         self.cold_blocks[:] = 0
         self.cold_free = self.num_cold
         self.cold_exact = True
@@ -1143,6 +1150,44 @@ def select_rows_layers(pools: Sequence[PagePool], src_rows: Sequence[int]) -> No
     new_lens[:, :n], new_hw[:, :n] = lens[:, r], hw[:, r]
     for l, (p, k) in enumerate(zip(pools, need.tolist())):
         p._selected(new_lens[l], new_hw[l], int(k))
+
+
+def _one_device(pools: list) -> bool:
+    """Distinct GPU pools of one device, all quantised or none: a model's layers take one launch."""
+    g = pools[0]
+    quant = getattr(g, "quantized", False)
+    return (g.device.type == "cuda" and len({id(p) for p in pools}) == len(pools)
+            and all(p.device == g.device and getattr(p, "quantized", False) == quant for p in pools))
+
+
+def crop_layers(pools: Sequence[PagePool], batch: int, max_length: int) -> None:
+    """``PagePool.crop(batch, max_length)`` on every pool, in one launch when no pool has pages to
+    re-open (pages shared after a selection, blocks quantised past the new length)."""
+    pools = list(pools)
+    if len(pools) > 1 and batch > 0 and _one_device(pools):
+        quant = getattr(pools[0], "quantized", False)
+        if (quant or not any(p.shared for p in pools)) and _gpu_backend().crop_layers_(
+                [p.seq_lens for p in pools], [p.lens for p in pools],
+                [p.cold_blocks if quant else None for p in pools], [p.page_size for p in pools], batch,
+                max(int(max_length), 0)):
+            return
+    for p in pools:
+        p.crop(batch, max_length)
+
+
+def reset_layers(pools: Sequence[PagePool]) -> None:
+    """``PagePool.reset()`` on every pool, in one launch for a model's GPU pools."""
+    pools = list(pools)
+    if len(pools) < 2 or not _one_device(pools):
+        for p in pools:
+            p.reset()
+        return
+    backend = _gpu_backend()
+    packed = [p._packed(backend) for p in pools]
+    colds = [h[2] for h in packed] if getattr(pools[0], "quantized", False) else []
+    backend.reset_layers_([h[1] for h in packed], colds, pools[0].key_pages)
+    for p in pools:
+        p._emptied()
 
 
 class _HostOps:
