@@ -2232,6 +2232,22 @@ int run_stream(const barq_kv_pool* pool, const void* ks, const void* vs, int64_t
           lean_m = balanced_chunks(aligned, resident);
       }
     }
+    // Past one round of them, one-page tiles still beat the rounds kernel while they are small or the
+    // launch stores many tokens (its last tiles move each twice).  Gathers, us, rounds kernel -> lean:
+    // 16 KiB tiles (64 vectors a row) 40.5 -> 36.0 at 23 tiles a CU, 182 -> 176 at 128; 32 KiB
+    // 31.8 -> 28.6 at 9, 40.2 -> 37.8 at 12, 94.0 -> 94.4 at 32, ragged rows 42.2 -> 43.0 at 16;
+    // 64 KiB 31.4 -> 30.3 at 4.2, 40.9 -> 39.8 at 6, 54.8 -> 57.2 at 8.  Appends of 256 to 2048
+    // tokens with their gather: 64 KiB 55.2 -> 48.3 at 7.5, 85.5 -> 75.7 at 11, 102 -> 97 at 15;
+    // 32 KiB 54.1 -> 52.4 at 16.
+    if (lean_ppt == 0 && (P * lpp) % 4 == 0) {
+      const int64_t nu = P * lpp / 4;
+      const int64_t tiles_1 = 2 * batch * ((span + P - 1) / P);
+      const int64_t limit = nu == 4 ? kI32Max / ncu : tokens > P ? 16 : nu == 8 ? 12 : 6;
+      if ((nu == 4 || nu == 8 || nu == 16) && tiles_1 <= limit * ncu) {
+        lean_ppt = 1;
+        lean_nu = nu;
+      }
+    }
   }
 
   // Rows kernel: a gather launch the wave-uniform mapping does not take, in 16-byte vectors, whose
