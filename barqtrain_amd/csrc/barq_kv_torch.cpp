@@ -439,11 +439,20 @@ void advance(int64_t* L, int64_t* W, int64_t batch, int64_t tokens) {
   }
 }
 
-// An append from the shadow's state where it is exact, else from the device's.
+// Whether work on the stream is being recorded (or cannot be told not to be): a replay's row state is the
+// device's, not the shadow's of now.
+bool recording(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// An append from the shadow's state where it is exact, else (and in a graph) from the device's.
 int append_step(const barq_kv_pool& p, const at::Tensor& k, const at::Tensor& v, const int64_t* L, const int64_t* W,
                 const int64_t* rows, int64_t free_count, bool free_exact, void* stream) {
   const int64_t batch = k.size(0), tokens = k.size(2);
-  if (free_exact && batch <= 64) {
+  if (free_exact && batch <= 64 && !recording(stream)) {
     int32_t l32[64], w32[64], r32[64];
     for (int64_t i = 0; i < batch; ++i) {
       const int64_t r = rows ? rows[i] : i;

@@ -47,3 +47,37 @@ def test_known_appends_match_device_reads(hip, H, D, P, dtype, rows):
         for a, b in zip(known.gather(rows), plain.gather(rows)):
             assert torch.equal(a.view(torch.uint8), b.view(torch.uint8)), step
     assert known.errors() == plain.errors() == 0
+
+
+def test_captured_appends_follow_the_device_state(hip):
+    """A graph's append (and append_rows) stores at the rows' lengths of each replay."""
+    gen = torch.Generator().manual_seed(9)
+    make = lambda: PagePool(max_batch=3, max_blocks=8, page_size=4, kv_heads=2, head_dim=64, dtype=torch.bfloat16,
+                            device="cuda")
+    pool, eager = make(), make()
+    k, v = (hf_layout(3, 2, 1, 64, torch.bfloat16, gen).cuda() for _ in range(2))
+
+    def step(p):
+        p.append(k, v)
+        p.append_rows([2, 0], k[:2], v[:2])
+
+    for p in (pool, eager):
+        step(p)
+    state = [(a.copy(), a) for a in (pool.lens, pool.hw)], pool.free_count
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(pool)
+    for copy, a in state[0]:  # nothing of the recording has run
+        a[:] = copy
+    pool.free_count = state[1]
+    for it in range(5):
+        k.copy_(hf_layout(3, 2, 1, 64, torch.bfloat16, gen))
+        v.copy_(hf_layout(3, 2, 1, 64, torch.bfloat16, gen))
+        graph.replay()
+        step(eager)
+        torch.cuda.synchronize()
+        for name in ("block_table", "seq_lens", "high_water"):
+            assert torch.equal(getattr(pool, name), getattr(eager, name)), (it, name)
+        for a, b in zip(pool.gather(3, int(eager.lens.max())), eager.gather(3)):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16)), it
+    assert pool.errors() == eager.errors() == 0
