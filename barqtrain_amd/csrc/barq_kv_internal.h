@@ -16,6 +16,15 @@ int append_known(const barq_kv_pool* pool, const void* key_states, const void* v
                  int64_t tokens, int64_t stride_b, int64_t stride_h, int64_t stride_t, const int32_t* rows,
                  const int32_t* seq_lens, const int32_t* high_water, int64_t free_top, void* stream);
 
+// The append of BARQ_KV_QUANT_DIRECT to rows [0, batch) that are all empty (length and mark 0), for a
+// caller that knows so and the tops of both free stacks; with key_out / value_out also
+// barq_kv_gather_cold of the `tokens` positions.  BARQ_KV_ERR_UNSUPPORTED, nothing launched, for what
+// the kernel does not take, stacks that hold too few pages included.
+int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* key_states,
+                      const void* value_states, int64_t batch, int64_t tokens, int64_t stride_b, int64_t stride_h,
+                      int64_t stride_t, void* key_out, void* value_out, int64_t osb, int64_t osh, int64_t oss,
+                      int64_t free_top, int64_t cold_top, void* stream);
+
 // barq_kv_crop of rows [0, batch) of n pools, whose row lengths are at seq_lens[i].
 int crop_layers(int32_t* const* seq_lens, int64_t n, int64_t batch, int64_t max_length, void* stream);
 

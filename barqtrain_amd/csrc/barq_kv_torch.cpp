@@ -298,21 +298,48 @@ void pool_compress_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, 
   check_status(barq_kv_compress(&p, &c, batch, current_stream(pool[0])), "pool_compress_");
 }
 
-// Append of any number of tokens, quantising what passes the window as it is stored; false (nothing
-// launched) when the pool or the states have a form the kernels do not take.
-bool pool_append_cold_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
-                       at::Tensor key_states, at::Tensor value_states) {
+// Whether work on the stream is being recorded (or cannot be told not to be): a replay's row state is the
+// device's, not the shadow's of now.
+bool recording(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
+// An append of any number of tokens that quantises past the window as it stores (BARQ_KV_QUANT_DIRECT).
+// tops: (free pages, free cold pages) of a caller that knows them and that every row is empty, else
+// none.  Returns 0 when the kernels do not take the call (nothing changed), 1 when appended, 2 when out
+// ((key, value), or empty) was also filled with the rows' `tokens` positions.
+int64_t pool_append_cold_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
+                          at::Tensor key_states, at::Tensor value_states, std::vector<at::Tensor> out,
+                          c10::optional<std::pair<int64_t, int64_t>> tops) {
   barq_kv_pool p = pool_from(pool);
   barq_kv_cold c = cold_from(p, pool[0], cold, window);
   check_states(p, pool[0], key_states, value_states);
+  const int64_t batch = key_states.size(0), tokens = key_states.size(2);
+  TORCH_CHECK(out.empty() || out.size() == 2, "out: nothing, or (key, value)");
+  if (!out.empty()) check_out(p, pool[0], out[0], out[1], batch, tokens);
   c10::DeviceGuard guard(pool[0].device());
-  const int rc = barq_kv_update_cold(&p, &c, key_states.data_ptr(), value_states.data_ptr(), key_states.size(0),
-                                     key_states.size(2), key_states.stride(0), key_states.stride(1),
-                                     key_states.stride(2), nullptr, nullptr, 0, 0, 0, 0, BARQ_KV_QUANT_DIRECT,
-                                     current_stream(pool[0]));
-  if (rc == BARQ_KV_ERR_UNSUPPORTED) return false;
+  void* stream = current_stream(pool[0]);
+  if (tops && batch > 0 && tokens > 0 && !recording(stream)) {
+    const bool fill = !out.empty();
+    const int rc = barq_internal::append_fresh_cold(
+        &p, &c, key_states.data_ptr(), value_states.data_ptr(), batch, tokens, key_states.stride(0),
+        key_states.stride(1), key_states.stride(2), fill ? out[0].data_ptr() : nullptr,
+        fill ? out[1].data_ptr() : nullptr, fill ? out[0].stride(0) : 0, fill ? out[0].stride(1) : 0,
+        fill ? out[0].stride(2) : 0, tops->first, tops->second, stream);
+    if (rc != BARQ_KV_ERR_UNSUPPORTED) {
+      check_status(rc, "pool_append_cold_");
+      return fill ? 2 : 1;
+    }
+  }
+  const int rc = barq_kv_update_cold(&p, &c, key_states.data_ptr(), value_states.data_ptr(), batch, tokens,
+                                     key_states.stride(0), key_states.stride(1), key_states.stride(2), nullptr,
+                                     nullptr, 0, 0, 0, 0, BARQ_KV_QUANT_DIRECT, stream);
+  if (rc == BARQ_KV_ERR_UNSUPPORTED) return 0;
   check_status(rc, "pool_append_cold_");
-  return true;
+  return 1;
 }
 
 void pool_gather_cold(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
@@ -437,15 +464,6 @@ void advance(int64_t* L, int64_t* W, int64_t batch, int64_t tokens) {
     L[r] += tokens;
     W[r] = std::max(W[r], L[r]);
   }
-}
-
-// Whether work on the stream is being recorded (or cannot be told not to be): a replay's row state is the
-// device's, not the shadow's of now.
-bool recording(void* stream) {
-  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing((hipStream_t)stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
-  (void)hipGetLastError();
-  return true;
 }
 
 // An append from the shadow's state where it is exact, else (and in a graph) from the device's.

@@ -738,12 +738,12 @@ class QuantPagePool(PagePool):
         self._quantised(batch, frontier, moved)
 
     def _append_direct(self, tensors: list[torch.Tensor], rows: slice, key_states: torch.Tensor,
-                       value_states: torch.Tensor) -> bool:
+                       value_states: torch.Tensor, out: Sequence[torch.Tensor] = ()) -> int:
         """A checked append of `rows` (the rows of `tensors`) in one go, blocks past the window
         quantised from the states themselves (BARQ_KV_QUANT_DIRECT): no chunks, and hot pages only
-        for what stays hot.  False, nothing changed, when the free hot pages do not cover those at
-        once (chunks also use the pages that quantised blocks return) or the kernels do not take
-        the geometry."""
+        for what stays hot.  0, nothing changed, when the free hot pages do not cover those at once
+        (chunks also use the pages that quantised blocks return) or the kernels do not take the
+        geometry; 2 when `out` (the whole of rows that were empty) was filled too; else 1."""
         tokens, P = key_states.shape[2], self.page_size
         lens, hw, cold = self.lens[rows], self.hw[rows], self.cold_blocks[rows]
         ends = lens + tokens
@@ -751,17 +751,20 @@ class QuantPagePool(PagePool):
         mapped = -(-hw // P)
         last = -(-ends // P)
         if int(np.maximum(last - np.maximum(mapped, frontier), 0).sum()) > self.free_count:
-            return False
+            return 0
         k, v = self._compatible_pair(key_states, value_states)
-        if not self._ops().pool_append_cold_(tensors, self.cold_tensors, self.window, k, v):
-            return False
+        empty = self.free_exact and self.cold_exact and not hw.any()
+        done = self._ops().pool_append_cold_(tensors, self.cold_tensors, self.window, k, v, list(out),
+                                             (self.free_count, self.cold_free) if empty else None)
+        if not done:
+            return 0
         moved = int(np.maximum(frontier - cold, 0).sum())
         self.free_count += moved - int(np.maximum(last - mapped, 0).sum())
         self.cold_free -= moved
         np.maximum(cold, frontier, out=cold)
         lens += tokens
         np.maximum(hw, lens, out=hw)
-        return True
+        return done
 
     def _check_chunked(self, batch: int, tokens: int, max_length: Optional[int],
                        rows: Optional[np.ndarray] = None) -> None:
@@ -836,6 +839,12 @@ class QuantPagePool(PagePool):
         self._check_states(key_states, value_states)
         batch, _, tokens, _ = key_states.shape
         if tokens > self.chunk:
+            if batch and self.on_gpu and out is None and seq_out is None and flags == 0 and not self.hw[:batch].any():
+                self._check_chunked(batch, tokens, max_length)
+                new = self._new_out(batch, tokens)
+                done = self._append_direct(self.tensors, slice(0, batch), key_states, value_states, new)
+                if done:
+                    return new if done == 2 else self.gather(batch, out=new)
             self.append(key_states, value_states, max_length)
             return self.gather(batch, seq_out, out, flags)
         need = self.check_append(batch, tokens, max_length)
