@@ -25,6 +25,15 @@ int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
                       int64_t stride_t, void* key_out, void* value_out, int64_t osb, int64_t osh, int64_t oss,
                       int64_t free_top, int64_t cold_top, void* stream);
 
+// barq_kv_update_cold (no BARQ_KV_SEQ_FROM_DEVICE) for a caller that knows the rows' lengths and marks
+// exactly, and the free stack's top after the call's compress; BARQ_KV_ERR_UNSUPPORTED, nothing
+// launched, for calls its one-launch update does not take.
+int update_cold_known(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* key_states,
+                      const void* value_states, int64_t batch, int64_t tokens, int64_t stride_b, int64_t stride_h,
+                      int64_t stride_t, void* key_out, void* value_out, int64_t seq_out, int64_t osb, int64_t osh,
+                      int64_t oss, int64_t flags, const int32_t* seq_lens, const int32_t* high_water,
+                      int64_t free_top, void* stream);
+
 // barq_kv_crop of rows [0, batch) of n pools, whose row lengths are at seq_lens[i].
 int crop_layers(int32_t* const* seq_lens, int64_t n, int64_t batch, int64_t max_length, void* stream);
 

@@ -1320,8 +1320,19 @@ struct UpdateArgs {
   FastDiv div_page;
 };
 
-template <int KIND, int LPP>
-__global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(LPP <= 2 ? 5 : 3))) update_cold_lanes_kernel(const UpdateArgs u) {
+// The row state of a caller that knows it exactly (barq_internal::update_cold_known): no tile reads it
+// from the device, none arrives, and the first workgroup commits.  An arrival is a round trip to a
+// counter that the tile's first wave makes before its loads: 16 rows of 648 positions (8 x 128 bf16,
+// 64 MB) took 17.9 us with arrivals and take 15.5 without.  (Six waves a SIMD spill, 19.5 us; four or
+// three tiles a CU at a time, 16.1 - 16.3; up to 12 positions a tile, cut evenly, 19.2.)
+struct KnownRows {
+  int32_t len[kWave];
+  int32_t hw[kWave];
+  int32_t top;
+};
+
+template <int KIND, int LPP, bool KNOWN>
+__device__ __forceinline__ void update_cold_tile(const UpdateArgs& u, const KnownRows* ks) {
   using V = Vec<KIND, 8>;
   using E = Elem<KIND>;
   using Bits = typename E::Bits;
@@ -1341,28 +1352,31 @@ __global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_pe
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
 
   // The launch's starting state (batch <= 64: one row per lane).
-  const int len = p.seq_lens[b];
-  const int hw = p.high_water[b];
+  const int len = KNOWN ? ks->len[b] : p.seq_lens[b];
+  const int hw = KNOWN ? ks->hw[b] : p.high_water[b];
   const int stored = p.block_table[(int64_t)b * mb + j];
   // The extent (longest row + tokens) matters only to a block reaching past its row's new end:
   // the others hold data at every position and skip the batch-wide read (every tile reading the
   // same lengths serialises on one L2 channel).
   int S = a.seq_out;
-  if (a.from_device && pos0 + P > len + T)
+  if (!KNOWN && a.from_device && pos0 + P > len + T)
     S = min(barq_commit::wave_max(lane < a.batch ? p.seq_lens[lane] + T : 0), a.seq_out);
   const barq_commit::NewBlocks nb = barq_commit::new_blocks(len, hw, T, mb, u.div_page);
   const bool fresh_block = j >= nb.first && j < nb.first + nb.count;
   int newpage = -1;
   if (fresh_block) {
-    const int top = p.ctrl[BARQ_KV_CTRL_FREE_TOP];
-    const int base = barq_commit::wave_sum(
-        lane < b ? barq_commit::new_blocks(p.seq_lens[lane], p.high_water[lane], T, mb, u.div_page).count : 0);
+    const int top = KNOWN ? ks->top : p.ctrl[BARQ_KV_CTRL_FREE_TOP];
+    const int rl = lane < b ? (KNOWN ? ks->len[lane] : p.seq_lens[lane]) : 0;
+    const int rh = lane < b ? (KNOWN ? ks->hw[lane] : p.high_water[lane]) : 0;
+    const int base = barq_commit::wave_sum(lane < b ? barq_commit::new_blocks(rl, rh, T, mb, u.div_page).count : 0);
     const int idx = top - 1 - (base + j - nb.first);
     newpage = idx >= 0 ? checked_id(p.free_pages[idx], p.num_pages) : -1;
   }
-  __builtin_amdgcn_s_waitcnt(0);  // every wave holds its metadata before the tile arrives
-  __syncthreads();
-  if (wave == 0) barq_commit::arrive_and_commit(p, u.nsub, a.batch, T, a.seq_out, u.div_page);
+  if constexpr (!KNOWN) {
+    __builtin_amdgcn_s_waitcnt(0);  // every wave holds its metadata before the tile arrives
+    __syncthreads();
+    if (wave == 0) barq_commit::arrive_and_commit(p, u.nsub, a.batch, T, a.seq_out, u.div_page);
+  }
   if (pos0 >= S) return;  // uniform
 
   const bool old_block = pos0 < hw;  // mapped before this append
@@ -1466,6 +1480,27 @@ __global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_pe
           if (t0 + i < end) __builtin_nontemporal_store(typename V::Out(0), (typename V::Out*)(o + (int64_t)i * a.oss + ocol[c]));
     }
   }
+}
+
+template <int KIND, int LPP>
+__global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(LPP <= 2 ? 5 : 3))) update_cold_lanes_kernel(const UpdateArgs u) {
+  update_cold_tile<KIND, LPP, false>(u, nullptr);
+}
+
+// The commit follows the first tile's data: no tile reads what it writes (a block of new positions takes
+// its page from the stack, whose entries stay).
+template <int KIND, int LPP>
+__global__ void __launch_bounds__(kGatherThreads) __attribute__((amdgpu_waves_per_eu(LPP <= 2 ? 5 : 3))) update_cold_known_kernel(const UpdateArgs u, const KnownRows ks) {
+  update_cold_tile<KIND, LPP, true>(u, &ks);
+  if (blockIdx.x != 0 || threadIdx.x >= kWave) return;
+  const barq_kv_pool& p = u.g.p;
+  const int lane = threadIdx.x, batch = u.g.batch;
+  const int len = lane < batch ? ks.len[lane] : 0, hw = lane < batch ? ks.hw[lane] : 0;
+  const int news = barq_commit::wave_sum(
+      lane < batch ? barq_commit::new_blocks(len, hw, u.tokens, (int)p.max_blocks, u.div_page).count : 0);
+  const int idx = ks.top - 1 - lane;
+  barq_commit::commit_from_lanes(p, batch, u.tokens, u.g.seq_out, u.div_page, len, hw, ks.top,
+                                 news > 0 && idx >= 0 ? p.free_pages[idx] : -1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1772,6 +1807,17 @@ const void* fresh_blocks_fn_t(int nv) {
 }
 
 template <int KIND>
+const void* update_fn_t(int lpp, bool known) {
+  if (known)
+    return lpp == 1   ? (const void*)&update_cold_known_kernel<KIND, 1>
+           : lpp == 2 ? (const void*)&update_cold_known_kernel<KIND, 2>
+                      : (const void*)&update_cold_known_kernel<KIND, 4>;
+  return lpp == 1   ? (const void*)&update_cold_lanes_kernel<KIND, 1>
+         : lpp == 2 ? (const void*)&update_cold_lanes_kernel<KIND, 2>
+                    : (const void*)&update_cold_lanes_kernel<KIND, 4>;
+}
+
+template <int KIND>
 int launch_gather(int ve, int lpp, dim3 grid, GatherArgs* a, hipStream_t s) {
   const void* fn = (const void*)&gather_cold_kernel<KIND, 1>;
   if constexpr (KIND != BARQ_KV_FP32) {  // 8 two-byte elements: a 16-byte vector
@@ -1837,7 +1883,7 @@ int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t 
 // only ever stores the one value a device gives.
 int resident_tiles(const void* fn, int slot) {
   constexpr int kMaxDevices = 64;
-  constexpr int kSlots = 6;
+  constexpr int kSlots = 12;
   static std::atomic<int> cached[kSlots][kMaxDevices];  // 0 = not queried yet
   int dev = 0;
   if (slot < 0 || slot >= kSlots || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
@@ -1883,7 +1929,8 @@ int append_direct(const barq_kv_pool* pool, const barq_kv_cold* cold, const void
 
 int update_cold_fused(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* ks, const void* vs,
                       int64_t batch, int64_t tokens, int64_t sb, int64_t sh, int64_t st, void* ko, void* vo,
-                      int64_t seq_out, int64_t osb, int64_t osh, int64_t oss, int64_t flags, void* stream) {
+                      int64_t seq_out, int64_t osb, int64_t osh, int64_t oss, int64_t flags, void* stream,
+                      const KnownRows* known = nullptr) {
   if (!cold_ok(pool, cold) || pool->elem_bytes != 2 || cold->element_type == BARQ_KV_FP32) return -1;
   if (batch < 1 || batch > kWave || batch > pool->max_batch || tokens < 1 || tokens > cold->window) return -1;
   const int64_t P = pool->page_size, H = pool->kv_heads, D = pool->head_dim;
@@ -1933,15 +1980,12 @@ int update_cold_fused(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
   u.nsub = (int32_t)std::min<int64_t>(tiles, BARQ_KV_CTRL_SUBCOUNTERS);
   u.div_page = FastDiv::make((uint32_t)P);
   const bool f16 = cold->element_type == BARQ_KV_FP16;
-  const void* fn = lpp == 1   ? (f16 ? (const void*)&update_cold_lanes_kernel<BARQ_KV_FP16, 1>
-                                     : (const void*)&update_cold_lanes_kernel<BARQ_KV_BF16, 1>)
-                   : lpp == 2 ? (f16 ? (const void*)&update_cold_lanes_kernel<BARQ_KV_FP16, 2>
-                                     : (const void*)&update_cold_lanes_kernel<BARQ_KV_BF16, 2>)
-                              : (f16 ? (const void*)&update_cold_lanes_kernel<BARQ_KV_FP16, 4>
-                                     : (const void*)&update_cold_lanes_kernel<BARQ_KV_BF16, 4>);
-  const int64_t resident = resident_tiles(fn, (lpp == 1 ? 0 : lpp == 2 ? 1 : 2) * 2 + (f16 ? 1 : 0));
+  const void* fn = f16 ? update_fn_t<BARQ_KV_FP16>(lpp, known != nullptr) : update_fn_t<BARQ_KV_BF16>(lpp, known != nullptr);
+  const int64_t resident = resident_tiles(fn, ((lpp == 1 ? 0 : lpp == 2 ? 1 : 2) * 2 + (f16 ? 1 : 0)) * 2 + (known ? 1 : 0));
   u.spaced = resident > 0 && tiles <= resident ? 1 : 0;
-  void* args[] = {&u};
+  KnownRows rows{};
+  if (known) rows = *known;
+  void* args[] = {&u, &rows};
   return hipLaunchKernel(fn, dim3((uint32_t)tiles), dim3(kGatherThreads), args, 0, (hipStream_t)stream) == hipSuccess
              ? BARQ_KV_OK
              : BARQ_KV_ERR_LAUNCH;
@@ -2122,6 +2166,25 @@ int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
                          (hipStream_t)stream) == hipSuccess
              ? BARQ_KV_OK
              : BARQ_KV_ERR_LAUNCH;
+}
+
+int update_cold_known(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* ks, const void* vs, int64_t batch,
+                      int64_t tokens, int64_t sb, int64_t sh, int64_t st, void* ko, void* vo, int64_t seq_out,
+                      int64_t osb, int64_t osh, int64_t oss, int64_t flags, const int32_t* seq_lens,
+                      const int32_t* high_water, int64_t free_top, void* stream) {
+  if ((flags & ~(int64_t)BARQ_KV_NO_COMPRESS) || !seq_lens || !high_water) return BARQ_KV_ERR_INVALID;
+  if (batch < 1 || batch > kWave) return BARQ_KV_ERR_UNSUPPORTED;
+  if (!pool || free_top < 0 || free_top > pool->num_pages) return BARQ_KV_ERR_INVALID;
+  KnownRows rows{};
+  for (int64_t r = 0; r < batch; ++r) {
+    rows.len[r] = seq_lens[r];
+    rows.hw[r] = high_water[r];
+    if (rows.len[r] < 0 || rows.hw[r] < rows.len[r]) return BARQ_KV_ERR_INVALID;
+  }
+  rows.top = (int32_t)free_top;
+  const int rc = update_cold_fused(pool, cold, ks, vs, batch, tokens, sb, sh, st, ko, vo, seq_out, osb, osh, oss, flags,
+                                   stream, &rows);
+  return rc < 0 ? BARQ_KV_ERR_UNSUPPORTED : rc;
 }
 
 }  // namespace barq_internal

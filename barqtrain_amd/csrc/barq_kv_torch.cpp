@@ -652,9 +652,21 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
     at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
     ko = both[0];
     vo = both[1];
-    rc = barq_kv_update_cold(&p, &c, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2),
-                             ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2),
-                             flags | (moved == 0 ? BARQ_KV_NO_COMPRESS : 0), stream);
+    const int64_t f = flags | (moved == 0 ? BARQ_KV_NO_COMPRESS : 0);
+    rc = BARQ_KV_ERR_UNSUPPORTED;
+    if (flags == 0 && free_exact && batch <= 64 && tokens <= c.window && !recording(stream)) {
+      int32_t l32[64], w32[64];
+      for (int64_t r = 0; r < batch; ++r) {
+        l32[r] = (int32_t)L[r];
+        w32[r] = (int32_t)W[r];
+      }
+      rc = barq_internal::update_cold_known(&p, &c, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1),
+                                            k.stride(2), ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0),
+                                            ko.stride(1), ko.stride(2), f, l32, w32, free_count + moved, stream);
+    }
+    if (rc == BARQ_KV_ERR_UNSUPPORTED)
+      rc = barq_kv_update_cold(&p, &c, k.data_ptr(), v.data_ptr(), batch, tokens, k.stride(0), k.stride(1), k.stride(2),
+                               ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2), f, stream);
   } else {
     rc = append_step(p, k, v, L, W, nullptr, free_count, free_exact, stream);
     if (rc == BARQ_KV_OK && moved > 0) rc = barq_kv_compress(&p, &c, batch, stream);
