@@ -624,8 +624,8 @@ void reset_layers_(const std::vector<at::Tensor>& pools, const std::vector<at::T
 
 // pool_step_ for a pool with a cold store, of at most `chunk` tokens: also the blocks that leave the
 // window (cold_blocks: the rows' leading quantised ones, updated in place), whose compress is
-// launched only when there are any.  Returns (key_out, value_out, pages taken, longest row, blocks
-// quantised).
+// launched only when there are any, or into a graph.  Returns (key_out, value_out, pages taken,
+// longest row, blocks quantised).
 std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
     const at::Tensor& handle, const at::Tensor& cold, const at::Tensor& pages, at::Tensor k, at::Tensor v,
     py::buffer lens, py::buffer hw, py::buffer cold_blocks, int64_t free_count, bool free_exact, int64_t cold_free,
@@ -647,14 +647,16 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
   if (moved > cold_free) return {ko, vo, -2, 0, 0};
   c10::DeviceGuard guard(pages.device());
   void* stream = current_stream(pages);
+  const bool graph = recording(stream);
+  const bool compress = moved > 0 || graph;  // a replay's rows may have blocks that leave the window
   int rc;
   if (gather) {
     at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
     ko = both[0];
     vo = both[1];
-    const int64_t f = flags | (moved == 0 ? BARQ_KV_NO_COMPRESS : 0);
+    const int64_t f = flags | (compress ? 0 : BARQ_KV_NO_COMPRESS);
     rc = BARQ_KV_ERR_UNSUPPORTED;
-    if (flags == 0 && free_exact && batch <= 64 && tokens <= c.window && !recording(stream)) {
+    if (flags == 0 && free_exact && batch <= 64 && tokens <= c.window && !graph) {
       int32_t l32[64], w32[64];
       for (int64_t r = 0; r < batch; ++r) {
         l32[r] = (int32_t)L[r];
@@ -669,7 +671,7 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
                                ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2), f, stream);
   } else {
     rc = append_step(p, k, v, L, W, nullptr, free_count, free_exact, stream);
-    if (rc == BARQ_KV_OK && moved > 0) rc = barq_kv_compress(&p, &c, batch, stream);
+    if (rc == BARQ_KV_OK && compress) rc = barq_kv_compress(&p, &c, batch, stream);
   }
   check_status(rc, gather ? "pool_update_cold_" : "pool_append_");
   for (int64_t r = 0; r < batch; ++r) C[r] = std::max(C[r], frontier(r));

@@ -146,6 +146,11 @@ class PagePool:
     def _ops(self):
         return _gpu_backend() if self.on_gpu else _HostOps
 
+    def _recording(self) -> bool:
+        """Whether the current stream is being captured: the rows' state when a graph is replayed is the
+        device's, so nothing may be left out of it on the host shadow's word."""
+        return self.on_gpu and torch.cuda.is_current_stream_capturing()
+
     def _index_tensor(self, rows: Sequence[int]) -> torch.Tensor:
         """Row indices as int32 on the pool's device, copied from pinned memory without waiting
         for the stream (a plain host-to-device copy would synchronise it)."""
@@ -732,7 +737,7 @@ class QuantPagePool(PagePool):
         k, v = self._compatible_pair(key_states, value_states)
         ops = self._ops()
         ops.pool_append_(self.tensors, k, v)
-        if moved:  # else no block leaves the window: no compress launch
+        if moved or self._recording():  # else no block leaves the window: no compress launch
             ops.pool_compress_(self.tensors, self.cold_tensors, self.window, batch)
         self._advance(batch, tokens, need)
         self._quantised(batch, frontier, moved)
@@ -854,7 +859,7 @@ class QuantPagePool(PagePool):
         seq = int((self.lens[:batch] + tokens).max()) if seq_out is None else int(seq_out)
         ko, vo = out if out is not None else self._new_out(batch, seq)
         k, v = self._compatible_pair(key_states, value_states)
-        skip = NO_COMPRESS if moved == 0 else 0  # no block leaves the window: no compress launch
+        skip = NO_COMPRESS if moved == 0 and not self._recording() else 0  # no block leaves the window
         self._ops().pool_update_cold_(self.tensors, self.cold_tensors, self.window, k, v, ko, vo, seq, flags | skip)
         self._advance(batch, tokens, need)
         self._quantised(batch, frontier, moved)
