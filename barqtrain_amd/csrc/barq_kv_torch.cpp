@@ -517,7 +517,7 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t> pool_step_(const at::Tensor
     at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
     ko = both[0];
     vo = both[1];
-    if (flags == 0 && free_exact && batch <= 64) {
+    if (flags == 0 && free_exact && batch <= 64 && !recording(current_stream(pages))) {
       // The shadow is exact: the launch takes the row state in its arguments.
       int32_t l32[64], w32[64];
       for (int64_t r = 0; r < batch; ++r) {

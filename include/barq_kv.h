@@ -190,8 +190,12 @@ int barq_kv_update(const barq_kv_pool* pool, const void* key_states, const void*
  * gives wrong pages and lengths, as a wrong block table would).  The same results and pool state
  * as barq_kv_update, from a launch that reads none of that state on the device and commits it
  * without waiting for every tile (a small launch then ends with its copies, not after two
- * dependent counter round trips).  Launches outside the kernel's shapes (more than 64 rows, tiles
- * not all resident at once, other geometries) run barq_kv_update.  It replaces the same
+ * dependent counter round trips).  The state is an argument of the launch: in a graph, every replay
+ * would run with the recording's values, so record barq_kv_update there.  Batches of up to 64 rows
+ * in 16-byte vectors take it when the launch is of page-aligned lean tiles (token rows of 64, 128 or
+ * 256 vectors, all tiles resident at once, or one-page tiles in few rounds), or of token rows of
+ * other sizes whose pages are whole waves' loads (page_size * vectors a multiple of 64); every other
+ * launch runs barq_kv_update.  It replaces the same
  * reference path as barq_kv_update, the per-call paged_kv_append_ + current_tensors of
  * python/barqtrain/kv_cache.py:93-142, for callers that track their lengths on the host
  * (BarqPagedKVCacheLayer's shadow, kv_cache.py:150-153 read without a sync).

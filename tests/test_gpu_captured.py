@@ -108,3 +108,30 @@ def test_recorded_fp8_updates_quantise_on_replay(hip, out):
             take_shadow(pool, eager)
             same(pool, eager, B, it)
     assert int(eager.cold_blocks.min()) > 2
+
+
+# 16 and 80 vectors a row (the rows kernel), 128: resident at once, and one-page tiles of several rounds
+@pytest.mark.parametrize("H,D,B,length", [(2, 64, 3, 60), (5, 128, 3, 60), (8, 128, 3, 60), (8, 128, 64, 200)])
+def test_recorded_updates_follow_the_device_state(hip, H, D, B, length):
+    gen = torch.Generator().manual_seed(H * B)
+    make = lambda: PagePool(max_batch=B, max_blocks=16, page_size=16, kv_heads=H, head_dim=D, dtype=BF16, device="cuda")
+    pool, eager = make(), make()
+    k, v = states(gen, B, 1, H, D)
+    first, some = states(gen, B, length, H, D), states(gen, 2, 5, H, D)
+    for p in (pool, eager):
+        p.append(*first)
+    got = []
+    graph = record([pool], [eager], lambda: got.extend(pool.update(k, v)))
+    for p in (pool, eager):
+        p.free_rows([1])
+        p.crop(B, length // 2)
+        p.append_rows([0, 2], *some)
+    for it in range(6):
+        for x, new in zip((k, v), states(gen, B, 1, H, D)):
+            x.copy_(new)
+        graph.replay()
+        for a, b in zip(got, eager.update(k, v)):
+            assert torch.equal(a[:, :, :b.shape[2]].view(torch.int16), b.view(torch.int16)), it
+        take_shadow(pool, eager)
+        same(pool, eager, B, it)
+        assert torch.equal(pool.block_table, eager.block_table)
