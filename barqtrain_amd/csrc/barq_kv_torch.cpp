@@ -575,7 +575,7 @@ barq_kv_cold one_cold(const at::Tensor& handle) {
 // A crop of rows [0, batch) of a model's layers in one launch: the pools' row lengths, their host
 // shadows (updated in place) and, for pools with cold stores, the rows' leading quantised blocks.
 // False, nothing done, when a crop would re-open a quantised block (colds[i][r] * page_sizes[i] past
-// the row's new length).
+// the row's new length), or a replay of the graph being recorded could.
 bool crop_layers_(const std::vector<at::Tensor>& seq_lens, const std::vector<py::buffer>& lens,
                   const std::vector<c10::optional<py::buffer>>& colds, const std::vector<int64_t>& page_sizes,
                   int64_t batch, int64_t max_length) {
@@ -584,6 +584,9 @@ bool crop_layers_(const std::vector<at::Tensor>& seq_lens, const std::vector<py:
               "crop_layers_: one entry per pool");
   std::vector<int32_t*> device(n);
   std::vector<int64_t*> host(n);
+  TORCH_CHECK(seq_lens[0].is_cuda(), "row lengths must be on a GPU");
+  c10::DeviceGuard guard(seq_lens[0].device());
+  const bool graph = recording(current_stream(seq_lens[0]));
   for (size_t i = 0; i < n; ++i) {
     const at::Tensor& t = seq_lens[i];
     TORCH_CHECK(t.is_cuda() && t.get_device() == seq_lens[0].get_device() && t.scalar_type() == at::kInt &&
@@ -592,12 +595,12 @@ bool crop_layers_(const std::vector<at::Tensor>& seq_lens, const std::vector<py:
     device[i] = t.data_ptr<int32_t>();
     host[i] = shadow(lens[i], batch);
     if (colds[i].has_value()) {
+      if (graph) return false;
       const int64_t* c = shadow(*colds[i], batch);
       for (int64_t r = 0; r < batch; ++r)
         if (c[r] > std::min(host[i][r], max_length) / page_sizes[i]) return false;
     }
   }
-  c10::DeviceGuard guard(seq_lens[0].device());
   check_status(barq_internal::crop_layers(device.data(), (int64_t)n, batch, max_length, current_stream(seq_lens[0])),
                "crop_layers_");
   for (int64_t* L : host)

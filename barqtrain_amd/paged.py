@@ -1176,7 +1176,8 @@ def _one_device(pools: list) -> bool:
 
 def crop_layers(pools: Sequence[PagePool], batch: int, max_length: int) -> None:
     """``PagePool.crop(batch, max_length)`` on every pool, in one launch when no pool has pages to
-    re-open (pages shared after a selection, blocks quantised past the new length)."""
+    re-open (pages shared after a selection, blocks quantised past the new length, or in a graph any
+    quantised ones: a replay's rows may hold such blocks)."""
     pools = list(pools)
     if len(pools) > 1 and batch > 0 and _one_device(pools):
         quant = getattr(pools[0], "quantized", False)

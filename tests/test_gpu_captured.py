@@ -2,11 +2,14 @@
 shadow said when they were recorded: every replay is compared with a twin pool that makes the same
 calls eagerly -- lengths, marks, stack tops and the bits that a gather reads."""
 
+import types
+
 import pytest
 import torch
 
 from kvgen import hf_layout
 
+from barqtrain_amd.kv_cache import create_paged_kv_cache
 from barqtrain_amd.paged import SEQ_FROM_DEVICE, PagePool, QuantPagePool
 
 pytestmark = pytest.mark.gpu
@@ -135,3 +138,30 @@ def test_recorded_updates_follow_the_device_state(hip, H, D, B, length):
         take_shadow(pool, eager)
         same(pool, eager, B, it)
         assert torch.equal(pool.block_table, eager.block_table)
+
+
+def test_recorded_fp8_crops_reopen_quantised_blocks(hip):
+    """A cache's crop recorded where it re-opens nothing, replayed where quantised blocks lie past it."""
+    B, layers, gen = 3, 2, torch.Generator().manual_seed(4)
+    caches = [create_paged_kv_cache(types.SimpleNamespace(num_hidden_layers=layers), max_batch_size=B, max_cache_len=240,
+                                    page_size=16, kv_quant="fp8", residual_window=32) for _ in range(2)]
+    pools, eager = ([], [])
+    first, more, one = states(gen, B, 70), states(gen, B, 64), states(gen, B, 1)
+    for l in range(layers):
+        for cache, group in zip(caches, (pools, eager)):
+            cache.update(*first, l)
+            group.append(cache.layers[l].pool)
+    graph = record(pools, eager, lambda: caches[0].crop(40))
+    for it in range(3):
+        for l in range(layers):
+            for cache in caches:
+                cache.update(*more, l)
+        assert int(eager[0].cold_blocks.min()) * 16 > 40
+        graph.replay()
+        caches[1].crop(40)
+        for l in range(layers):
+            take_shadow(pools[l], eager[l])
+            same(pools[l], eager[l], B, it)
+            for a, b in zip(caches[0].update(*one, l), caches[1].update(*one, l)):
+                assert torch.equal(a.view(torch.int16), b.view(torch.int16)), it
+            same(pools[l], eager[l], B, it)
