@@ -310,7 +310,9 @@ bool recording(void* stream) {
 // An append of any number of tokens that quantises past the window as it stores (BARQ_KV_QUANT_DIRECT).
 // tops: (free pages, free cold pages) of a caller that knows them and that every row is empty, else
 // none.  Returns 0 when the kernels do not take the call (nothing changed), 1 when appended, 2 when out
-// ((key, value), or empty) was also filled with the rows' `tokens` positions.
+// ((key, value), or empty) was also filled with the rows' `tokens` positions.  Not recorded into a graph:
+// it takes its hot pages at once, for rows whose state at a replay nobody has checked them for (chunks
+// return pages as they go).
 int64_t pool_append_cold_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window,
                           at::Tensor key_states, at::Tensor value_states, std::vector<at::Tensor> out,
                           c10::optional<std::pair<int64_t, int64_t>> tops) {
@@ -322,7 +324,8 @@ int64_t pool_append_cold_(std::vector<at::Tensor> pool, std::vector<at::Tensor> 
   if (!out.empty()) check_out(p, pool[0], out[0], out[1], batch, tokens);
   c10::DeviceGuard guard(pool[0].device());
   void* stream = current_stream(pool[0]);
-  if (tops && batch > 0 && tokens > 0 && !recording(stream)) {
+  if (recording(stream)) return 0;
+  if (tops && batch > 0 && tokens > 0) {
     const bool fill = !out.empty();
     const int rc = barq_internal::append_fresh_cold(
         &p, &c, key_states.data_ptr(), value_states.data_ptr(), batch, tokens, key_states.stride(0),

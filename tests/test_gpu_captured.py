@@ -165,3 +165,20 @@ def test_recorded_fp8_crops_reopen_quantised_blocks(hip):
             for a, b in zip(caches[0].update(*one, l), caches[1].update(*one, l)):
                 assert torch.equal(a.view(torch.int16), b.view(torch.int16)), it
             same(pools[l], eager[l], B, it)
+
+
+@pytest.mark.parametrize("update", [False, True])
+def test_recorded_long_fp8_appends_fit_where_chunks_fit(hip, update):
+    """A prompt recorded over empty rows, replayed behind 47 tokens in a pool that holds just what chunks
+    need (five pages a row: three hot ones before it, three after it, four during it)."""
+    B, gen = 3, torch.Generator().manual_seed(5)
+    pool, eager = (quant_pool(B, chunk=16, num_pages=5 * B) for _ in range(2))
+    prompt, first = states(gen, B, 64), states(gen, B, 47)
+    graph = record([pool], [eager], lambda: pool.update(*prompt) if update else pool.append(*prompt))
+    for p in (pool, eager):
+        p.append(*first)
+    graph.replay()
+    eager.append(*prompt)
+    take_shadow(pool, eager)
+    same(pool, eager, B, update)
+    assert eager.lens.tolist() == [111] * B
