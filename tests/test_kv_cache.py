@@ -3,6 +3,7 @@ package through the reference import path ``barqtrain``.  CPU tensors, no GPU ne
 
 import types
 
+import pytest
 import torch
 
 from barqtrain.kv_cache import (
@@ -144,3 +145,25 @@ def test_decode_step_strides_of_hf_accepted_without_copy():
     prefill_v = torch.randn(3, 2, 21, 128)                 # genuinely different layouts: copied
     k, v = PagePool._compatible_pair(prefill_k, prefill_v)
     assert k.stride() == v.stride() and k.is_contiguous()
+
+
+@pytest.mark.parametrize("args,kwargs,length", [((4,), {}, 4), ((-2,), {}, 5), ((), {"tokens_to_remove": -2}, 5),
+                                                ((), {"tokens_to_remove": 4}, 4), ((), {"max_length": 3}, 3),
+                                                ((), {"max_length": -3}, 4)])
+def test_cache_crop_by_position_and_by_either_name(args, kwargs, length):
+    cache = create_paged_kv_cache(ThreeLayerText(), max_batch_size=1, max_cache_len=8, page_size=4)
+    keys = torch.arange(14, dtype=torch.float32).view(1, 1, 7, 2)
+    for layer in range(3):
+        cache.update(keys, -keys, layer)
+    cache.crop(*args, **kwargs)
+    for layer in cache.layers:
+        assert layer.get_seq_length() == length
+        assert torch.equal(layer.current_tensors()[0], keys[:, :, :length])
+
+
+def test_cache_crop_needs_one_length():
+    cache = create_paged_kv_cache(ThreeLayerText(), max_batch_size=1, max_cache_len=8, page_size=4)
+    with pytest.raises(TypeError):
+        cache.crop()
+    with pytest.raises(TypeError):
+        cache.crop(1, max_length=1)
