@@ -9,7 +9,9 @@ import torch
 
 from kvgen import hf_layout
 
+from barqtrain_amd import kv_cache
 from barqtrain_amd.kv_cache import create_paged_kv_cache
+from barqtrain_amd.paged import crop_layers
 
 pytestmark = pytest.mark.gpu
 H, D, B, BF16 = 2, 64, 3, torch.bfloat16
@@ -81,3 +83,26 @@ def test_cache_crop_after_a_selection_reopens_shared_pages(hip):
         gk, gv = cache.update(k, k, l)
         assert torch.equal(gk, torch.cat([wk, k], 2)) and torch.equal(gv, torch.cat([wv, k], 2))
         assert cache.layers[l].pool.errors() == 0
+
+
+@pytest.mark.parametrize("quant", [False, True])
+@pytest.mark.parametrize("uneven", [False, True])
+@pytest.mark.parametrize("count", [-1, -3, -69, -500])
+def test_cache_crop_by_a_negative_count_is_every_layers_crop(hip, monkeypatch, quant, uneven, count):
+    """Tokens to remove: one launch where the layers hold the same length."""
+    one, each = filled(5, quant), filled(5, quant)
+    if uneven:
+        k = hf_layout(B, H, 2, D, BF16, torch.Generator().manual_seed(3)).cuda()
+        one.update(k, k, 2), each.update(k, k, 2)
+    together = []
+    monkeypatch.setattr(kv_cache, "crop_layers", lambda *a: together.append(a) or crop_layers(*a))
+    one.crop(count)
+    assert len(together) == (not uneven)
+    for layer in each.layers:
+        layer.crop(count)
+    for a, b in zip(one.layers, each.layers):
+        assert a.get_seq_length() == b.get_seq_length() == max(70 + 2 * (uneven and a is one.layers[2]) + count, 0)
+        assert a.pool.seq_lens.tolist() == b.pool.seq_lens.tolist() == a.pool.lens.tolist()
+        assert a.pool.ctrl[[0, 2]].tolist() == b.pool.ctrl[[0, 2]].tolist()
+        for x, y in zip(a.current_tensors(), b.current_tensors()):
+            assert torch.equal(x.view(torch.int16), y.view(torch.int16))
