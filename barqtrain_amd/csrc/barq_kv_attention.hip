@@ -1378,11 +1378,13 @@ __global__ __launch_bounds__(NT) void attention_merge_kernel(const AttnArgs a) {
   }
 }
 
-// Resident workgroups of THREADS threads of a kernel on the current device, at most kMaxWaves
-// (cached per instantiation and device; host threads may race on the cache, which only ever
-// stores the one value a device gives); `fallback` when the runtime cannot tell.
-template <int THREADS, typename K>
-int resident_blocks(K kernel, int fallback) {
+// Resident workgroups of THREADS threads of a kernel on the current device, at most kMaxWaves;
+// `fallback` when the runtime cannot tell.  Cached per kernel and device: the kernel is a template
+// argument, since kernels share their pointer's type and not their registers (a flat kernel of 16
+// query rows holds one wave a SIMD, one of 4 rows two).  Host threads may race on the cache, which
+// only ever stores the one value a device gives.
+template <int THREADS, auto Kernel>
+int resident_blocks(int fallback) {
   constexpr int kMaxDevices = 64;
   static std::atomic<int> cached[kMaxDevices];  // 0 = not queried yet
   int dev = 0;
@@ -1391,18 +1393,12 @@ int resident_blocks(K kernel, int fallback) {
   if (blocks == 0) {
     int cus = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, THREADS, 0) != hipSuccess)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, Kernel, THREADS, 0) != hipSuccess)
       return fallback;
     blocks = std::min(std::max(cus * per_cu, 1), kMaxWaves);
     if (dev >= 0 && dev < kMaxDevices) cached[dev].store(blocks, std::memory_order_relaxed);
   }
   return blocks;
-}
-
-// Resident waves of a one-wave-workgroup kernel.
-template <typename K>
-int resident_waves(K kernel) {
-  return resident_blocks<kWave>(kernel, kMaxWaves);
 }
 
 template <int HD, int E, int R, bool U, typename OutT, bool COLD>
@@ -1420,11 +1416,11 @@ hipError_t launch_typed(AttnArgs a, bool merge, hipStream_t stream) {
     // 28.4).
     // Workgroups a pair: as many as are resident at once with the others' (the kernel decides per
     // row how many it uses), at most kMaxSplit; the pair counts in ctrl bound the pairs.
-    auto* split_any = attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitAny>;
+    constexpr auto split_any = &attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitAny>;
     const int64_t chunks = (a.max_seq + kBlock - 1) / kBlock;
     const int64_t nsplit =
         pairs > 0 && pairs <= BARQ_KV_CTRL_PAIR_SLOTS && chunks >= 2 * pair_part_chunks<R>()
-            ? std::min<int64_t>(kMaxSplit, resident_blocks<kPairWaves * kWave>(split_any, 0) / pairs)
+            ? std::min<int64_t>(kMaxSplit, resident_blocks<kPairWaves * kWave, split_any>(0) / pairs)
             : 1;
     int64_t max_chunks = R > 1 || pairs < kPairMinPairs        ? kPairMaxChunks
                          : COLD || pairs < 2 * kPairMinPairs ? kPairMaxChunksR1
@@ -1449,9 +1445,9 @@ hipError_t launch_typed(AttnArgs a, bool merge, hipStream_t stream) {
     // (Head size 256 keeps the flat schedule there: 1 x 30000 positions, G 4: 24.2 against 31.8 us.)
     if constexpr (HD <= 128) {
       if (a.range_chunks == 0 && pairs > 0 && pairs <= BARQ_KV_CTRL_PAIR_SLOTS) {
-        auto* split_long = attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitLong>;
+        constexpr auto split_long = &attention_pair_kernel<HD, E, R, OutT, COLD, kPairWaves, kSplitLong>;
         const int64_t nlong =
-            std::min<int64_t>(kMaxSplitLong, resident_blocks<kPairWaves * kWave>(split_long, 0) / pairs);
+            std::min<int64_t>(kMaxSplitLong, resident_blocks<kPairWaves * kWave, split_long>(0) / pairs);
         if (nlong > 2 && chunks <= nlong * kLongChunksPerPart) {
           hipLaunchKernelGGL(split_long, dim3((unsigned)(nlong * pairs)), dim3(kPairWaves * kWave), 0, stream, a);
           return hipGetLastError();
@@ -1459,8 +1455,8 @@ hipError_t launch_typed(AttnArgs a, bool merge, hipStream_t stream) {
       }
     }
   }
-  auto* k = attention_flat_kernel<HD, E, R, U, OutT, COLD>;
-  a.waves = resident_waves(k);
+  constexpr auto k = &attention_flat_kernel<HD, E, R, U, OutT, COLD>;
+  a.waves = resident_blocks<kWave, k>(kMaxWaves);
   hipLaunchKernelGGL(k, dim3((unsigned)a.waves), dim3(kWave), 0, stream, a);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess || !merge) return err;
