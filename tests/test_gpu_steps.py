@@ -2,6 +2,7 @@
 path; attention calls that must fall back to it; copies of a pool that has stepped."""
 
 import copy
+import types
 
 import numpy as np
 import pytest
@@ -11,6 +12,7 @@ from attn_ref import decode_attention_reference, within_tolerance
 from kvgen import hf_layout, to_bits
 from oracle.kv_quant_oracle import QuantLayerOracle
 
+from barqtrain_amd.kv_cache import BarqPagedKVCacheLayer, create_paged_kv_cache
 from barqtrain_amd.paged import PagedKVCapacityError, PagedKVPoolExhausted, PagePool, QuantPagePool
 
 pytestmark = pytest.mark.gpu
@@ -95,3 +97,37 @@ def test_attention_steps_and_their_fallbacks_agree(hip):
             assert out.shape == q.shape and torch.equal(out, outs[0])
             # one rounding to bf16 of sums within 2e-5
             assert within_tolerance(out.cpu().double().numpy(), want, 2.0 ** -8 + 2e-5, 2e-5)[0]
+
+
+def test_overridden_methods_of_layers_and_pools_are_called(hip):
+    """A layer's append (fused attention), a pool's update, append, crop and reset."""
+    calls = []
+
+    def counting(cls, *names):
+        def method(name):
+            return lambda self, *a, **kw: calls.append(name) or getattr(cls, name)(self, *a, **kw)
+        return type("Counting", (cls,), {name: method(name) for name in names})
+
+    k, v = (x.cuda() for x in kv(1, 2, 3, 64, torch.Generator().manual_seed(4)))
+    sub = counting(BarqPagedKVCacheLayer, "append")(max_batch_size=1, max_cache_len=32, fused_attention=True)
+    sub.update(k, v)
+    sub.update(k, v)
+    assert calls == ["append"] * 2 and sub.get_seq_length() == 6
+    layer = BarqPagedKVCacheLayer(max_batch_size=1, max_cache_len=32, fused_attention=True)
+    layer.update(k, v)
+    layer.append = lambda *a: calls.append("replaced") or type(layer).append(layer, *a)
+    layer.update(k, v)
+    assert calls[2:] == ["replaced"] and layer.get_seq_length() == 6
+    for pool_type in (PagePool, QuantPagePool):
+        cache = create_paged_kv_cache(types.SimpleNamespace(num_hidden_layers=2), max_batch_size=1, max_cache_len=64)
+        for l in range(2):
+            cache.update(k, v, l)
+            cache.layers[l].pool = counting(pool_type, "append", "update", "crop", "reset")(
+                max_batch=1, max_blocks=4, page_size=16, kv_heads=2, head_dim=64, dtype=BF16, device="cuda")
+        calls.clear()
+        for l, fused in enumerate((False, True)):
+            cache.layers[l].fused_attention = fused
+            cache.update(k, v, l)
+        cache.crop(1)
+        cache.reset()
+        assert [c for c in calls if c != "reset"] == ["update", "append", "crop", "crop"] and calls[-2:] == ["reset"] * 2
