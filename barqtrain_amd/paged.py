@@ -129,6 +129,10 @@ class PagePool:
         # A copy packs its own tensors and takes its own workspace.
         return {**self.__dict__, "_handle": None, "_attn_ws": None}
 
+    def __setstate__(self, state):
+        # Also a pool that was saved without these, or with its own tensors' addresses packed.
+        self.__dict__.update(state, _handle=None, _attn_ws=None)
+
     # ------------------------------------------------------------------ plumbing
     @property
     def on_gpu(self) -> bool:

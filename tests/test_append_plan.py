@@ -5,6 +5,8 @@ capacity error when a row would pass the limit."""
 
 from __future__ import annotations
 
+import pickle
+
 import numpy as np
 import pytest
 import torch
@@ -46,3 +48,18 @@ def test_plan_matches_per_row_restatement():
         assert need == _reference_need(lens[:batch], hw[:batch], T, P, mb)
         checked += 1
     assert checked > 500
+
+
+def test_a_pool_saved_without_its_packed_tensors_loads(monkeypatch):
+    """Pools pickled before these attributes were set from the start, or with addresses packed in them."""
+    pool = PagePool(max_batch=2, max_blocks=2, page_size=4, kv_heads=1, head_dim=4, dtype=torch.float32, device="cpu")
+    keys = torch.arange(24, dtype=torch.float32).view(2, 1, 3, 4)
+    pool.append(keys, -keys)
+    for extra in ({}, {"_handle": (0, torch.zeros(8))}):
+        state = {k: v for k, v in pool.__dict__.items() if k not in ("_handle", "_attn_ws")}
+        with monkeypatch.context() as m:
+            m.setattr(PagePool, "__getstate__", lambda self: {**state, **extra})
+            saved = pickle.dumps(pool)
+        loaded = pickle.loads(saved)
+        assert loaded._handle is None and loaded.attention_workspace(10).numel() >= 10
+        assert torch.equal(loaded.gather(2)[0], keys) and loaded.lens.tolist() == [3, 3]
