@@ -25,6 +25,10 @@ int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
                       int64_t stride_t, void* key_out, void* value_out, int64_t osb, int64_t osh, int64_t oss,
                       int64_t free_top, int64_t cold_top, void* stream);
 
+// barq_kv_compress for the lengths that rows [0, batch) reach after `ahead` more tokens, by a caller that
+// knows that the cold stack holds enough pages: a row's blocks are then taken by several workgroups.
+int compress_spread(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, int64_t ahead, void* stream);
+
 // barq_kv_update_cold (no BARQ_KV_SEQ_FROM_DEVICE) for a caller that knows the rows' lengths and marks
 // exactly, and the free stack's top after the call's compress; BARQ_KV_ERR_UNSUPPORTED, nothing
 // launched, for calls its one-launch update does not take.

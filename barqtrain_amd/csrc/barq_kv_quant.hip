@@ -15,6 +15,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include "barq_kv.h"
 #include <atomic>
@@ -296,18 +297,25 @@ __global__ void __launch_bounds__(kThreads) compress_kernel(const CompressArgs a
 }
 
 // ---------------------------------------------------------------------------------------------
-// Blocks quantised by whole workgroups, a wave to each (K or V, head) of a block: the compress of
-// pools whose pages divide into waves (quant_blocks_vectors below), and an append of any number
-// of tokens that quantises what passes the residual window straight from the input.
+// Blocks quantised by a wave to each (K or V, head) of a block: the compress of pools whose pages
+// divide into waves (quant_blocks_vectors below), and an append of any number of tokens that
+// quantises what passes the residual window straight from the input.
 //
 // A unit = one head of a block's K (or V), NV vectors of 16 bytes per lane: lane l holds column
 // l % vd (vd = vectors per head row) of tokens l / vd + i * 64 / vd.  Key maxima over the page's
 // tokens and value maxima over head_dim then cross lanes of one wave only -- no LDS, no barrier --
-// and a block's units are independent, so a workgroup of up to 16 waves takes a block in one round
-// trip of loads.  (One 256-thread workgroup per row, its blocks one after the other through LDS,
-// left 240 of 256 CUs idle on a batch of 16: 33 us for four pages a row.)
+// and units are independent, so a workgroup of up to 16 waves takes a block in one round trip of
+// loads.
 //
-// Tiles (row, i): i < nnew is the i-th block that receives new tokens -- a block the commit has
+// Quantised blocks lead every row (the attention kernels and a crop count on it), also when the cold
+// store runs out.  So in compress_blocks_kernel each row has one workgroup, which takes the pages of
+// the row's hot blocks with one atomic and quantises as many as it got, the first ones.  Where the
+// store cannot run out -- the append's plan below has counted, or the caller has (spread) --
+// quant_blocks_kernel spreads a row's blocks over workgroups.  16 rows of the 8 x 128 bf16 shape, one
+// page a row 10.7 us in order and 10.8 spread (launch and events included), four pages 20.7 and 11.4;
+// one workgroup of 256 threads a row, its blocks one after the other through LDS, took 14.6 and 35.9.
+//
+// Tiles (row, i): i < nnew is the i-th block that receives new tokens -- a block the plan has
 // just mapped to a cold page is quantised from the input, one that stays behind the frontier is
 // copied to its hot page, one that was hot before (the row's partial block, blocks a crop
 // re-opened) is quantised from its page and the input; i >= nnew are the row's older hot blocks.
@@ -315,12 +323,12 @@ __global__ void __launch_bounds__(kThreads) compress_kernel(const CompressArgs a
 // tops, which no other part of the launch moves the other way.
 //
 // Bound: HBM (the input read once, codes and scales written once), then the round trips of a
-// workgroup's only block.  A 16 x 1000-token prompt of the 8 x 128 bf16 shape: 24.7 us for 95 MB
+// workgroup's only block.  A 16 x 1000-token prompt of the 8 x 128 bf16 shape: 24.1 us for 95 MB
 // after a 6.8 us plan, against 16 chunks of an append and a compress each, 9.2 + 33 us.
 // ---------------------------------------------------------------------------------------------
 
-// Tiles per row that look for older hot blocks: a decode step has one such block every page_size
-// steps, an append of 64 tokens four (page size 16).
+// Tiles per row that look for older hot blocks: an append of 64 tokens pushes four out of the window
+// (page size 16).
 constexpr int kOldTiles = 4;
 
 struct QuantArgs {
@@ -588,7 +596,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(NV <=
         s_cold = c;
       }
       __syncthreads();
-      cp = s_cold;  // -1: no cold page left, the block stays hot
+      cp = s_cold;  // (-1, the block stays hot: not the pages that the plan or the caller counted)
     }
 #pragma unroll 1
     for (int u = wave; u < 2 * H; u += nwaves) {  // a wave's units: heads of K, then of V
@@ -630,11 +638,110 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(NV <=
   if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);
 }
 
+// Compress of one row, a pass of kScan entries a lane at a time (every wave scans for itself).
+constexpr int kScan = 4;
+
+template <int KIND, int NV>
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) compress_blocks_kernel(const QuantArgs a) {
+  using V = typename RawC<16>::T;
+  __shared__ int s_top, s_avail;
+  const barq_kv_pool& p = a.p;
+  const int b = (int)blockIdx.x;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int nwaves = (int)blockDim.x / kWave;
+  const int P = (int)p.page_size, H = (int)p.kv_heads, mb = (int)p.max_blocks;
+  const int len = p.seq_lens[b] + a.ahead;
+  const int frontier = min(len > a.c.window ? (int)a.div_page.div((uint32_t)(len - a.c.window)) : 0,
+                           min(ceil_div_fd(max(p.high_water[b], len), a.div_page), mb));
+  int32_t* row = p.block_table + (int64_t)b * mb;
+  int err = 0;
+  for (int j0 = 0; j0 < frontier; j0 += kScan * kWave) {
+    int found[kScan];      // the lane's hot page, of block j0 + kWave * k + lane
+    uint64_t hot[kScan];   // lanes that have one
+    int count = 0;
+#pragma unroll
+    for (int k = 0; k < kScan; ++k) {
+      const int j = j0 + kWave * k + lane;
+      found[k] = j < frontier ? row[j] : -1;
+    }
+#pragma unroll
+    for (int k = 0; k < kScan; ++k) {
+      found[k] = checked_id(found[k], p.num_pages);
+      if (found[k] >= 0 && p.page_shares && p.page_shares[found[k]] != 0) found[k] = -1;
+      hot[k] = __builtin_amdgcn_ballot_w64(found[k] >= 0);
+      count += __builtin_popcountll(hot[k]);
+    }
+    if (count == 0) continue;  // uniform
+    if (threadIdx.x == 0) {
+      const int before = atomicSub(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], count);
+      int avail = 0;
+      if ((int64_t)before > a.c.num_cold) err |= BARQ_KV_ERRBIT_BAD_INDEX;
+      else avail = min(max(before, 0), count);
+      if (avail < count) {
+        atomicAdd(&p.ctrl[BARQ_KV_CTRL_COLD_TOP], count - avail);
+        err |= err ? 0 : BARQ_KV_ERRBIT_POOL_EXHAUSTED;
+      }
+      s_top = before;
+      s_avail = avail;
+    }
+    __syncthreads();
+    const int avail = s_avail;
+    const int32_t* cold = a.c.free_cold + (s_top - 1);  // the q-th hot block takes cold[-q]
+    // Units (block, heads of K, then of V) dealt to the waves in turn.
+    int q = 0, u = wave;
+#pragma unroll
+    for (int k = 0; k < kScan; ++k) {
+      uint64_t left = hot[k];
+      for (; left != 0 && q < avail; ++q) {
+        const int l = __builtin_ctzll(left);
+        left &= left - 1;
+        if (u < 2 * H) {
+          const int hp = __builtin_amdgcn_readlane(found[k], l);
+          const int cp = checked_id(cold[-q], a.c.num_cold);
+#pragma unroll 1
+          for (; u < 2 * H; u += nwaves) {
+            const int kv = u >= H ? 1 : 0, h = u - kv * H;
+            V x[NV];
+            load_unit<KIND, NV>(a, b, kv, h, hp, 0, P, x);
+            if (cp >= 0) quantise_unit<KIND, NV>(a, kv, h, cp, x);
+          }
+        }
+        u -= 2 * H;
+      }
+    }
+    __syncthreads();  // every wave has read its hot pages, s_top and s_avail before they change
+    if (wave == 0) {
+      int first = 0;  // rank of the 64 entries' first hot block
+#pragma unroll
+      for (int k = 0; k < kScan; ++k) {
+        const int rank = first + __builtin_popcountll(hot[k] & ((1ull << lane) - 1));
+        first += __builtin_popcountll(hot[k]);
+        const int cp = found[k] >= 0 && rank < avail ? checked_id(cold[-rank], a.c.num_cold) : -1;
+        if (found[k] >= 0 && rank < avail && cp < 0) err |= BARQ_KV_ERRBIT_BAD_INDEX;
+        const uint64_t done = __builtin_amdgcn_ballot_w64(cp >= 0);
+        if (done == 0) continue;  // uniform
+        int slot = 0;
+        if (lane == 0) slot = atomicAdd(&p.ctrl[BARQ_KV_CTRL_FREE_TOP], __builtin_popcountll(done));
+        slot = __builtin_amdgcn_readfirstlane(slot) + __builtin_popcountll(done & ((1ull << lane) - 1));
+        if (cp >= 0) {
+          row[j0 + kWave * k + lane] = BARQ_KV_COLD_ENTRY(cp);
+          if (slot < p.num_pages) p.free_pages[slot] = found[k];
+          else err |= BARQ_KV_ERRBIT_BAD_INDEX;
+        }
+      }
+    }
+    if (avail < count) break;  // uniform: what follows stays hot too
+  }
+  if (err) atomicOr(&p.ctrl[BARQ_KV_CTRL_ERRORS], err);
+}
+
 // Commit of such an append, before its blocks are written: one workgroup maps every row's new
 // blocks -- those wholly before the window at the row's new end to cold pages, the rest to hot
 // pages, each ranked in (row, block) order on its stack -- and advances the rows.  If a row passes
-// its capacity or a stack holds too few pages, nothing changes but the error bits, and
-// ctrl[BARQ_KV_CTRL_APPEND_OK] = 0 tells the launch that follows.
+// its capacity or a stack holds too few pages -- the cold one also those of the rows' hot blocks that
+// leave the window -- nothing changes but the error bits, and ctrl[BARQ_KV_CTRL_APPEND_OK] = 0 tells
+// the launch that follows.
 struct AppendPlanArgs {
   barq_kv_pool p;
   ColdPtrs c;
@@ -649,14 +756,14 @@ __global__ void __launch_bounds__(kPlanThreads) append_plan_kernel(const AppendP
   __shared__ int s_scan[2][kPlanThreads / kWave];
   __shared__ int s_incl[2][kPlanThreads];  // rank ends of the chunk's rows: cold, hot
   __shared__ int s_first[2][kPlanThreads];
-  __shared__ int s_bad;
+  __shared__ int s_bad, s_old;
   const barq_kv_pool& p = a.p;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid / kWave;
   const int mb = (int)p.max_blocks;
   const int top = p.ctrl[BARQ_KV_CTRL_FREE_TOP];
   const int ctop = p.ctrl[BARQ_KV_CTRL_COLD_TOP];
-  if (tid == 0) s_bad = 0;
+  if (tid == 0) s_bad = s_old = 0;
   __syncthreads();
   // pass 0 counts, pass 1 maps
   for (int pass = 0; pass < 2; ++pass) {
@@ -726,6 +833,23 @@ __global__ void __launch_bounds__(kPlanThreads) append_plan_kernel(const AppendP
       __syncthreads();  // s_scan / s_incl / s_first are rewritten by the next chunk of rows
     }
     if (pass == 0) {
+      // Hot blocks that leave the window: at most the hot pages in use, and counted one by one only
+      // where the cold stack might not hold that many.
+      if (used[0] <= ctop && ctop - used[0] < (int)p.num_pages - top) {  // uniform
+        int old = 0;
+        for (int r = wave; r < a.batch; r += kPlanThreads / kWave) {
+          const int behind = p.seq_lens[r] + a.tokens - a.c.window;
+          const int n = min(min(behind > 0 ? (int)a.div_page.div((uint32_t)behind) : 0, ceil_div_fd(p.high_water[r], a.div_page)), mb);
+          const int32_t* row = p.block_table + (int64_t)r * mb;
+          for (int j = lane; j < n; j += kWave) {
+            const int page = checked_id(row[j], p.num_pages);
+            old += page >= 0 && (!p.page_shares || p.page_shares[page] == 0);
+          }
+        }
+        if (old > 0) atomicAdd(&s_old, old);
+        __syncthreads();
+        used[0] += s_old;
+      }
       if (used[0] > ctop || ctop > a.c.num_cold || used[1] > top || top > p.num_pages)
         err |= BARQ_KV_ERRBIT_POOL_EXHAUSTED;
       if (err) atomicOr(&s_bad, err);
@@ -1738,6 +1862,16 @@ const void* compress_fn(int64_t kind, int ve) {
 }
 
 template <int KIND>
+const void* compress_blocks_fn_t(int nv) {
+  switch (nv) {
+    case 1: return (const void*)&compress_blocks_kernel<KIND, 1>;
+    case 2: return (const void*)&compress_blocks_kernel<KIND, 2>;
+    case 4: return (const void*)&compress_blocks_kernel<KIND, 4>;
+    default: return (const void*)&compress_blocks_kernel<KIND, 8>;
+  }
+}
+
+template <int KIND>
 const void* quant_blocks_fn_t(int nv) {
   switch (nv) {
     case 1: return (const void*)&quant_blocks_kernel<KIND, 1>;
@@ -1747,7 +1881,7 @@ const void* quant_blocks_fn_t(int nv) {
   }
 }
 
-// 16-byte vectors per lane of one head of a page when quant_blocks_kernel takes the pool -- a head
+// 16-byte vectors per lane of one head of a page when the kernels above take the pool -- a head
 // row of a power of two of vectors, up to a wave's 64, and a head's page of 1, 2, 4 or 8 waves of
 // them -- every page, code and key-scale address aligned to its vector; else 0.
 int quant_blocks_vectors(const barq_kv_pool* p, const barq_kv_cold* c) {
@@ -1762,10 +1896,11 @@ int quant_blocks_vectors(const barq_kv_pool* p, const barq_kv_cold* c) {
   return nv == 1 || nv == 2 || nv == 4 || nv == 8 ? (int)nv : 0;
 }
 
-// Launches quant_blocks_kernel over `batch` rows: `tokens` already committed (append) or `ahead`.
+// Quantises blocks of `batch` rows: behind an append of `tokens`, already committed, or for the rows'
+// lengths `ahead` tokens on, in order or spread.
 int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, int nv, int64_t batch, int64_t tokens,
-                        int64_t ahead, const void* ks, const void* vs, int64_t sb, int64_t sh, int64_t st,
-                        hipStream_t stream) {
+                        int64_t ahead, bool spread, const void* ks, const void* vs, int64_t sb, int64_t sh,
+                        int64_t st, hipStream_t stream) {
   QuantArgs a;
   a.p = *pool;
   a.c = cold_ptrs(cold);
@@ -1784,11 +1919,15 @@ int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, int 
   a.vd_log2 = __builtin_ctzll((unsigned long long)vd);
   a.div_page = FastDiv::make((uint32_t)P);
   a.div_tiles = FastDiv::make((uint32_t)(nnew + kOldTiles));
-  const int64_t tiles = batch * (nnew + kOldTiles);
+  const bool tiled = tokens > 0 || spread;
+  const int64_t tiles = tiled ? batch * (nnew + kOldTiles) : batch;
   if (tiles > kI32Max) return BARQ_KV_ERR_INVALID;
-  const void* fn = cold->element_type == BARQ_KV_BF16   ? quant_blocks_fn_t<BARQ_KV_BF16>(nv)
-                   : cold->element_type == BARQ_KV_FP16 ? quant_blocks_fn_t<BARQ_KV_FP16>(nv)
-                                                        : quant_blocks_fn_t<BARQ_KV_FP32>(nv);
+  const auto fn_of = [&](auto kind) {
+    return tiled ? quant_blocks_fn_t<decltype(kind)::value>(nv) : compress_blocks_fn_t<decltype(kind)::value>(nv);
+  };
+  const void* fn = cold->element_type == BARQ_KV_BF16   ? fn_of(std::integral_constant<int, BARQ_KV_BF16>{})
+                   : cold->element_type == BARQ_KV_FP16 ? fn_of(std::integral_constant<int, BARQ_KV_FP16>{})
+                                                        : fn_of(std::integral_constant<int, BARQ_KV_FP32>{});
   const int threads = kWave * (int)std::min<int64_t>(16, 2 * pool->kv_heads);
   void* args[] = {&a};
   return hipLaunchKernel(fn, dim3((uint32_t)tiles), dim3((uint32_t)threads), args, 0, stream) == hipSuccess
@@ -1848,13 +1987,14 @@ int barq_kv_cold_reset(const barq_kv_pool* pool, const barq_kv_cold* cold, void*
 
 namespace {
 
-// barq_kv_compress for the lengths the rows [0, batch) will have after `ahead` more tokens.
-int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, int64_t ahead,
+// barq_kv_compress for the lengths the rows [0, batch) will have after `ahead` more tokens; spread: the
+// caller has counted enough cold pages.
+int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, int64_t ahead, bool spread,
                     void* stream) {
   if (!cold_ok(pool, cold) || batch < 0 || batch > pool->max_batch) return BARQ_KV_ERR_INVALID;
   if (batch == 0) return BARQ_KV_OK;
   if (const int nv = quant_blocks_vectors(pool, cold))
-    return launch_quant_blocks(pool, cold, nv, batch, 0, ahead, nullptr, nullptr, 0, 0, 0, (hipStream_t)stream);
+    return launch_quant_blocks(pool, cold, nv, batch, 0, ahead, spread, nullptr, nullptr, 0, 0, 0, (hipStream_t)stream);
   CompressArgs a;
   a.p = *pool;
   a.c = cold_ptrs(cold);
@@ -1923,7 +2063,7 @@ int append_direct(const barq_kv_pool* pool, const barq_kv_cold* cold, const void
   if (hipLaunchKernel((const void*)&append_plan_kernel, dim3(1), dim3(kPlanThreads), args, 0,
                       (hipStream_t)stream) != hipSuccess)
     return BARQ_KV_ERR_LAUNCH;
-  return launch_quant_blocks(pool, cold, nv, batch, tokens, 0, key_states, value_states, stride_b, stride_h, stride_t,
+  return launch_quant_blocks(pool, cold, nv, batch, tokens, 0, true, key_states, value_states, stride_b, stride_h, stride_t,
                              (hipStream_t)stream);
 }
 
@@ -1951,7 +2091,7 @@ int update_cold_fused(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
     return -1;
   const int lpp = (int)(hd8 / kWave);
   if (!(flags & BARQ_KV_NO_COMPRESS)) {
-    const int rc = compress_launch(pool, cold, batch, tokens, stream);
+    const int rc = compress_launch(pool, cold, batch, tokens, false, stream);
     if (rc != BARQ_KV_OK) return rc;
   }
   UpdateArgs u;
@@ -1996,7 +2136,7 @@ int update_cold_fused(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
 extern "C" {
 
 int barq_kv_compress(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, void* stream) {
-  return compress_launch(pool, cold, batch, 0, stream);
+  return compress_launch(pool, cold, batch, 0, false, stream);
 }
 
 int barq_kv_gather_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, void* key_out,
@@ -2166,6 +2306,10 @@ int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
                          (hipStream_t)stream) == hipSuccess
              ? BARQ_KV_OK
              : BARQ_KV_ERR_LAUNCH;
+}
+
+int compress_spread(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, int64_t ahead, void* stream) {
+  return compress_launch(pool, cold, batch, ahead, true, stream);
 }
 
 int update_cold_known(const barq_kv_pool* pool, const barq_kv_cold* cold, const void* ks, const void* vs, int64_t batch,

@@ -291,11 +291,14 @@ void pool_cold_reset_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold
   check_status(barq_kv_cold_reset(&p, &c, current_stream(pool[0])), "pool_cold_reset_");
 }
 
-void pool_compress_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window, int64_t batch) {
+// spread: the caller has counted enough cold pages (never for a graph's replays).
+void pool_compress_(std::vector<at::Tensor> pool, std::vector<at::Tensor> cold, int64_t window, int64_t batch, bool spread) {
   barq_kv_pool p = pool_from(pool);
   barq_kv_cold c = cold_from(p, pool[0], cold, window);
   c10::DeviceGuard guard(pool[0].device());
-  check_status(barq_kv_compress(&p, &c, batch, current_stream(pool[0])), "pool_compress_");
+  void* stream = current_stream(pool[0]);
+  check_status(spread ? barq_internal::compress_spread(&p, &c, batch, 0, stream) : barq_kv_compress(&p, &c, batch, stream),
+               "pool_compress_");
 }
 
 // Whether work on the stream is being recorded (or cannot be told not to be): a replay's row state is the
@@ -648,19 +651,28 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
   const StepPlan s = plan_step(p, L, W, batch, tokens, free_count, limit);
   if (s.need < 0) return {ko, vo, s.need, 0, 0};
   const auto frontier = [&](int64_t r) { return std::max<int64_t>(L[r] + tokens - c.window, 0) / p.page_size; };
-  int64_t moved = 0;
-  for (int64_t r = 0; r < batch; ++r) moved += std::max<int64_t>(frontier(r) - C[r], 0);
+  int64_t moved = 0, most = 0;  // blocks, of all rows and of one
+  for (int64_t r = 0; r < batch; ++r) {
+    const int64_t n = std::max<int64_t>(frontier(r) - C[r], 0);
+    moved += n;
+    most = std::max(most, n);
+  }
   if (moved > cold_free) return {ko, vo, -2, 0, 0};
   c10::DeviceGuard guard(pages.device());
   void* stream = current_stream(pages);
   const bool graph = recording(stream);
   const bool compress = moved > 0 || graph;  // a replay's rows may have blocks that leave the window
+  const bool spread = most > 1 && !graph;    // the cold pages of now are counted above
   int rc;
   if (gather) {
     at::Tensor both = at::empty({2, batch, p.kv_heads, s.worst, p.head_dim}, pages.options());
     ko = both[0];
     vo = both[1];
-    const int64_t f = flags | (compress ? 0 : BARQ_KV_NO_COMPRESS);
+    int64_t f = flags | (compress ? 0 : BARQ_KV_NO_COMPRESS);
+    if (spread && tokens <= c.window && !(flags & BARQ_KV_NO_COMPRESS)) {  // the blocks lie before the new tokens
+      check_status(barq_internal::compress_spread(&p, &c, batch, tokens, stream), "pool_update_cold_");
+      f |= BARQ_KV_NO_COMPRESS;
+    }
     rc = BARQ_KV_ERR_UNSUPPORTED;
     if (flags == 0 && free_exact && batch <= 64 && tokens <= c.window && !graph) {
       int32_t l32[64], w32[64];
@@ -677,7 +689,8 @@ std::tuple<at::Tensor, at::Tensor, int64_t, int64_t, int64_t> pool_step_cold_(
                                ko.data_ptr(), vo.data_ptr(), s.worst, ko.stride(0), ko.stride(1), ko.stride(2), f, stream);
   } else {
     rc = append_step(p, k, v, L, W, nullptr, free_count, free_exact, stream);
-    if (rc == BARQ_KV_OK && compress) rc = barq_kv_compress(&p, &c, batch, stream);
+    if (rc == BARQ_KV_OK && compress)
+      rc = spread ? barq_internal::compress_spread(&p, &c, batch, 0, stream) : barq_kv_compress(&p, &c, batch, stream);
   }
   check_status(rc, gather ? "pool_update_cold_" : "pool_append_");
   for (int64_t r = 0; r < batch; ++r) C[r] = std::max(C[r], frontier(r));
@@ -845,7 +858,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("pool_copy_rows_", &pool_copy_rows_, "Build rows of a fresh pool as copies of source rows");
   m.def("pool_select_rows_", &pool_select_rows_, "Rows become selected rows, sharing their full pages");
   m.def("pool_cold_reset_", &pool_cold_reset_, "Every page of a pool's fp8 cold store free");
-  m.def("pool_compress_", &pool_compress_, "Quantise blocks behind the residual window into the cold store");
+  m.def("pool_compress_", &pool_compress_, "Quantise blocks behind the residual window into the cold store", py::arg("pool"),
+        py::arg("cold"), py::arg("window"), py::arg("batch"), py::arg("spread") = false);
   m.def("pool_append_cold_", &pool_append_cold_, "Append tokens, quantising past the residual window as they are stored");
   m.def("pool_gather_cold", &pool_gather_cold, "Materialise rows of a pool with a cold store, dequantising");
   m.def("pool_update_cold_", &pool_update_cold_, "Append, compress, materialise (pool with a cold store)");

@@ -742,7 +742,7 @@ class QuantPagePool(PagePool):
         ops = self._ops()
         ops.pool_append_(self.tensors, k, v)
         if moved or self._recording():  # else no block leaves the window: no compress launch
-            ops.pool_compress_(self.tensors, self.cold_tensors, self.window, batch)
+            ops.pool_compress_(self.tensors, self.cold_tensors, self.window, batch, not self._recording())
         self._advance(batch, tokens, need)
         self._quantised(batch, frontier, moved)
 
@@ -952,7 +952,7 @@ class QuantPagePool(PagePool):
                 start = int(self.lens[row])
                 need = max(min(-(-(start + n) // P), self.max_blocks) - (-(-int(self.hw[row]) // P)), 0)
                 ops.pool_append_(one, k[i:i + 1, :, s0:s0 + n], v[i:i + 1, :, s0:s0 + n])
-                ops.pool_compress_(one, self.cold_tensors, self.window, 1)
+                ops.pool_compress_(one, self.cold_tensors, self.window, 1, not self._recording())
                 self.lens[row] = start + n
                 self.hw[row] = max(int(self.hw[row]), start + n)
                 frontier = max(start + n - self.window, 0) // P
@@ -1378,7 +1378,7 @@ class _HostOps:
         return y
 
     @staticmethod
-    def pool_compress_(t, cold, window, batch):
+    def pool_compress_(t, cold, window, batch, spread=False):
         kp, vp, bt, lens, hw, free, ctrl, shares = t
         kc, vc, ks, vs, free_cold, _ = cold
         P, MB = _HostOps._geometry(t)

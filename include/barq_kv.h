@@ -376,9 +376,9 @@ int barq_kv_cold_reset(const barq_kv_pool* pool, const barq_kv_cold* cold, void*
 
 /*
  * Rows [0, batch): every hot block wholly before the residual window is quantised into a cold
- * page taken from free_cold and its hot page returns to free_pages (in no fixed order).  A block
- * finding no cold page stays hot and sets BARQ_KV_ERRBIT_POOL_EXHAUSTED; a hot page another
- * block shares (page_shares) stays hot.  Rows without such a block cost next to nothing, so it can
+ * page taken from free_cold and its hot page returns to free_pages (in no fixed order).  When
+ * free_cold runs out, a row's later blocks stay hot -- its quantised blocks lead it -- and
+ * BARQ_KV_ERRBIT_POOL_EXHAUSTED is set; a hot page another block shares (page_shares) stays hot.  Rows without such a block cost next to nothing, so it can
  * run after every append (and inside a captured graph).
  */
 int barq_kv_compress(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t batch, void* stream);
@@ -408,12 +408,12 @@ int barq_kv_gather_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, void
  * a row needs ceil(window / page_size) + 1 of them whatever the prompt -- and then the gather, if
  * seq_out > 0 (key_out and value_out may be null when it is 0).  The cache reads the same
  * afterwards; cold and hot pages of new blocks come off their stacks in (row, block) order.  All or
- * nothing: when a row would pass its capacity or a stack holds too few pages for the new blocks, no
- * row changes and the error bits say why.  (A block that was hot before and finds no cold page stays
- * hot, as in barq_kv_compress.)  Hot pages must have one holder, as a selection over pools with cold
- * stores leaves them.  Takes pools whose head rows are a power of two of 16-byte vectors, up to 64,
- * with 64, 128, 256 or 512 vectors to a head's page, and addresses and strides that are multiples
- * of 16 bytes (codes and key scales: 16 / elem_bytes); others return BARQ_KV_ERR_UNSUPPORTED with
+ * nothing: when a row would pass its capacity or a stack holds too few pages for the new blocks (the
+ * cold one: and for the hot blocks that leave the window), no row changes and the error bits say why.
+ * Hot pages must have one holder, as a selection over pools with cold stores leaves them.  Takes pools
+ * whose head rows are a power of two of 16-byte vectors, up to 64, with 64, 128, 256 or 512 vectors to
+ * a head's page, and addresses and strides that are multiples of 16 bytes (codes and key scales: 16 /
+ * elem_bytes); others return BARQ_KV_ERR_UNSUPPORTED with
  * nothing launched. */
 #define BARQ_KV_NO_COMPRESS 4
 #define BARQ_KV_QUANT_DIRECT 8
