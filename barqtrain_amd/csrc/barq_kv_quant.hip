@@ -305,7 +305,11 @@ __global__ void __launch_bounds__(kThreads) compress_kernel(const CompressArgs a
 // l % vd (vd = vectors per head row) of tokens l / vd + i * 64 / vd.  Key maxima over the page's
 // tokens and value maxima over head_dim then cross lanes of one wave only -- no LDS, no barrier --
 // and units are independent, so a workgroup of up to 16 waves takes a block in one round trip of
-// loads.
+// loads.  The compress also takes heads whose page is more than eight waves' vectors, a unit then
+// being some of K's columns or some of V's tokens (split), and less than one wave's, a unit then being
+// several heads (packed).  Such pools' page of 16 rows, launch and events included, against the kernel
+// of any geometry: 2 x 128 at page 64 22.4 -> 12.0 us, 1 x 256 at page 32 18.0 -> 11.6, 1 x 128 at page
+// 128 30.6 -> 12.0; 8 x 64 at page 4 10.2 -> 8.9, 16 x 64 at page 2 10.2 -> 8.7.
 //
 // Quantised blocks lead every row (the attention kernels and a crop count on it), also when the cold
 // store runs out.  So in compress_blocks_kernel each row has one workgroup, which takes the pages of
@@ -340,6 +344,7 @@ struct QuantArgs {
   int32_t ahead;          // compress: tokens the rows are about to receive
   int32_t nnew;           // tiles per row of blocks that receive tokens
   int32_t vd_log2;        // vectors per head row
+  int32_t mode_log2;      // split units: units per head; packed units: vectors of a head's page
   FastDiv div_page;
   FastDiv div_tiles;      // nnew + kOldTiles
 };
@@ -352,17 +357,47 @@ __device__ __forceinline__ int opaque_lane() {
   return lane;
 }
 
+enum : int { kWholeUnit = 0, kSplitUnit = 1, kPackedUnit = 2 };
+
+// Where a lane's vectors of a unit lie: columns from col of tokens t0 + i * step.
+struct UnitLane {
+  int col, t0, step;
+  bool first;         // of the lanes that share a column
+  int vectors;        // of a row in the unit
+  int reach;          // lanes that share a column are less than this apart
+};
+
+// piece: which of a head's units a split one is.
+template <int KIND, int NV, int MODE>
+__device__ __forceinline__ UnitLane unit_lane(const QuantArgs& a, int kv, int piece) {
+  constexpr int VE = 16 / (int)sizeof(typename Elem<KIND>::Bits);
+  int lane = opaque_lane();
+  UnitLane l;
+  l.reach = MODE == kPackedUnit ? 1 << a.mode_log2 : kWave;
+  if constexpr (MODE == kPackedUnit) lane &= l.reach - 1;
+  const int vl = MODE == kSplitUnit && kv == 0 ? a.vd_log2 - a.mode_log2 : a.vd_log2;
+  l.vectors = 1 << vl;
+  l.col = (lane & (l.vectors - 1)) * VE;
+  l.t0 = lane >> vl;
+  l.step = kWave >> vl;
+  l.first = l.t0 == 0;
+  if constexpr (MODE == kSplitUnit) {
+    if (kv == 0) l.col += (piece << vl) * VE;
+    else l.t0 += piece * NV * l.step;
+  }
+  return l;
+}
+
 // Loads unit (kv, h) of the block whose positions start at s0: from hot page hp (if any), and
 // positions from len on -- the launch's tokens -- from the input.  Lane offsets fit 32 bits.
-template <int KIND, int NV>
+template <int KIND, int NV, int MODE = kWholeUnit>
 __device__ __forceinline__ void load_unit(const QuantArgs& a, int b, int kv, int h, int hp, int s0, int len,
-                                          typename RawC<16>::T (&x)[NV]) {
+                                          typename RawC<16>::T (&x)[NV], int piece = 0) {
   using Bits = typename Elem<KIND>::Bits;
   using V = typename RawC<16>::T;
   const barq_kv_pool& p = a.p;
-  const int lane = opaque_lane();
-  const int col = (lane & ((1 << a.vd_log2) - 1)) * (16 / (int)sizeof(Bits));
-  const int t0 = lane >> a.vd_log2, step = kWave >> a.vd_log2;
+  const UnitLane l = unit_lane<KIND, NV, MODE>(a, kv, piece);
+  const int col = l.col, t0 = l.t0, step = l.step;
   const int HD = (int)(p.kv_heads * p.head_dim), P = (int)p.page_size;
   const Bits* in = (const Bits*)a.in[kv] + ((int64_t)b * a.isb + (int64_t)h * a.ish + (int64_t)(s0 - len) * a.ist);
   const uint32_t ist = (uint32_t)a.ist;
@@ -427,17 +462,16 @@ struct NoEmit {
   __device__ void operator()(A&&...) const {}
 };
 
-template <int KIND, int NV, typename Emit = NoEmit>
+template <int KIND, int NV, int MODE = kWholeUnit, typename Emit = NoEmit>
 __device__ __forceinline__ void quantise_unit(const QuantArgs& a, int kv, int h, int cp,
-                                              const typename RawC<16>::T (&x)[NV], const Emit& emit = Emit()) {
+                                              const typename RawC<16>::T (&x)[NV], const Emit& emit = Emit(),
+                                              int piece = 0) {
   using M = Mag<KIND>;
   constexpr int VE = M::kPacked ? 8 : 4;  // elements of a vector; EW of a word
   constexpr int EW = VE / 4;
   const barq_kv_pool& p = a.p;
-  const int lane = opaque_lane();
-  const int vd = 1 << a.vd_log2;
-  const int col = (lane & (vd - 1)) * VE;
-  const int t0 = lane >> a.vd_log2, step = kWave >> a.vd_log2;
+  const UnitLane l = unit_lane<KIND, NV, MODE>(a, kv, piece);
+  const int col = l.col, t0 = l.t0, step = l.step;
   const int P = (int)p.page_size, H = (int)p.kv_heads, D = (int)p.head_dim;
   float inv[VE];      // keys: 2^-e of the columns' scale exponents e in [-127, 120] (products are exact)
   uint32_t top[NV];   // values: the vectors' token maxima
@@ -458,7 +492,7 @@ __device__ __forceinline__ void quantise_unit(const QuantArgs& a, int kv, int h,
         for (int i = 0; i < NV; ++i) m[w] = M::max2(m[w], M::finite(x[i][w]));
       }
     }
-    for (int o = vd; o < kWave; o <<= 1) {
+    for (int o = l.vectors; o < l.reach; o <<= 1) {
 #pragma unroll
       for (int w = 0; w < 4; ++w) m[w] = M::max2(m[w], (uint32_t)__shfl_xor((int)m[w], o, kWave));
     }
@@ -469,7 +503,7 @@ __device__ __forceinline__ void quantise_unit(const QuantArgs& a, int kv, int h,
       inv[e] = __uint_as_float((uint32_t)(127 - ex) << 23);
       sc.b[e] = (uint8_t)(ex + 127);
     }
-    if (lane < vd) *(typename CodeVec<VE>::Raw*)(a.c.key_scales + ((int64_t)cp * H + h) * D + col) = sc.v;
+    if (l.first) *(typename CodeVec<VE>::Raw*)(a.c.key_scales + ((int64_t)cp * H + h) * D + col) = sc.v;
     __builtin_memcpy(scales, sc.b, VE);
   } else {
     uint32_t all = 0;
@@ -488,7 +522,7 @@ __device__ __forceinline__ void quantise_unit(const QuantArgs& a, int kv, int h,
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       if constexpr (M::kPacked) top[i] = max(top[i] & 0xFFFFu, top[i] >> 16);
-      for (int o = 1; o < vd; o <<= 1) top[i] = max(top[i], (uint32_t)__shfl_xor((int)top[i], o, kWave));
+      for (int o = 1; o < l.vectors; o <<= 1) top[i] = max(top[i], (uint32_t)__shfl_xor((int)top[i], o, kWave));
       const int ex = group_exponent(M::value(top[i], 0));
       top[i] = (uint32_t)(127 - ex) << 23;  // 2^-e
       if (col == 0) vscales[(uint32_t)((t0 + i * step) * H)] = (uint8_t)(ex + 127);
@@ -641,7 +675,7 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(NV <=
 // Compress of one row, a pass of kScan entries a lane at a time (every wave scans for itself).
 constexpr int kScan = 4;
 
-template <int KIND, int NV>
+template <int KIND, int NV, int MODE = kWholeUnit>
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) compress_blocks_kernel(const QuantArgs a) {
   using V = typename RawC<16>::T;
   __shared__ int s_top, s_avail;
@@ -689,6 +723,8 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
     const int avail = s_avail;
     const int32_t* cold = a.c.free_cold + (s_top - 1);  // the q-th hot block takes cold[-q]
     // Units (block, heads of K, then of V) dealt to the waves in turn.
+    const int packed = MODE == kPackedUnit ? kWave >> a.mode_log2 : 1;  // heads of a unit
+    const int units = MODE == kSplitUnit ? H << a.mode_log2 : MODE == kPackedUnit ? (H + packed - 1) / packed : H;
     int q = 0, u = wave;
 #pragma unroll
     for (int k = 0; k < kScan; ++k) {
@@ -696,18 +732,22 @@ __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4))) 
       for (; left != 0 && q < avail; ++q) {
         const int l = __builtin_ctzll(left);
         left &= left - 1;
-        if (u < 2 * H) {
+        if (u < 2 * units) {
           const int hp = __builtin_amdgcn_readlane(found[k], l);
           const int cp = checked_id(cold[-q], a.c.num_cold);
 #pragma unroll 1
-          for (; u < 2 * H; u += nwaves) {
-            const int kv = u >= H ? 1 : 0, h = u - kv * H;
+          for (; u < 2 * units; u += nwaves) {
+            const int kv = u >= units ? 1 : 0, n = u - kv * units;
+            const int piece = MODE == kSplitUnit ? n & ((1 << a.mode_log2) - 1) : 0;
+            const int h = MODE == kSplitUnit    ? n >> a.mode_log2
+                          : MODE == kPackedUnit ? min(n * packed + (lane >> a.mode_log2), H - 1)  // past the last: it again
+                                                : n;
             V x[NV];
-            load_unit<KIND, NV>(a, b, kv, h, hp, 0, P, x);
-            if (cp >= 0) quantise_unit<KIND, NV>(a, kv, h, cp, x);
+            load_unit<KIND, NV, MODE>(a, b, kv, h, hp, 0, P, x, piece);
+            if (cp >= 0) quantise_unit<KIND, NV, MODE>(a, kv, h, cp, x, NoEmit(), piece);
           }
         }
-        u -= 2 * H;
+        u -= 2 * units;
       }
     }
     __syncthreads();  // every wave has read its hot pages, s_top and s_avail before they change
@@ -1227,7 +1267,7 @@ __global__ void __launch_bounds__(kFreshWaves * kWave) __attribute__((amdgpu_wav
   if (to_cold && id >= 0) {  // uniform
     constexpr int VE = 16 / (int)sizeof(Bits);
     if (out) {  // uniform
-      quantise_unit<KIND, NV>(a, kv, h, id, x, [&](int t, int col, const uint32_t (&w)[VE / 4], const uint32_t (&ks)[VE / 4], uint32_t vs) {
+      quantise_unit<KIND, NV, kWholeUnit>(a, kv, h, id, x, [&](int t, int col, const uint32_t (&w)[VE / 4], const uint32_t (&ks)[VE / 4], uint32_t vs) {
         V v;
         if constexpr (KIND == BARQ_KV_FP32) {
           typename Vec<KIND, VE>::CodeU c, k;
@@ -1861,9 +1901,16 @@ const void* compress_fn(int64_t kind, int ve) {
                                 : compress_fn_t<BARQ_KV_FP32>(ve);
 }
 
+// How a compress takes a pool: vectors per lane of a unit (0: not at all) and the kind of units.
+struct QuantUnits {
+  int nv = 0, mode = kWholeUnit, log2 = 0;
+};
+
 template <int KIND>
-const void* compress_blocks_fn_t(int nv) {
-  switch (nv) {
+const void* compress_blocks_fn_t(const QuantUnits& q) {
+  if (q.mode == kSplitUnit) return (const void*)&compress_blocks_kernel<KIND, 8, kSplitUnit>;
+  if (q.mode == kPackedUnit) return (const void*)&compress_blocks_kernel<KIND, 1, kPackedUnit>;
+  switch (q.nv) {
     case 1: return (const void*)&compress_blocks_kernel<KIND, 1>;
     case 2: return (const void*)&compress_blocks_kernel<KIND, 2>;
     case 4: return (const void*)&compress_blocks_kernel<KIND, 4>;
@@ -1881,24 +1928,35 @@ const void* quant_blocks_fn_t(int nv) {
   }
 }
 
-// 16-byte vectors per lane of one head of a page when the kernels above take the pool -- a head
-// row of a power of two of vectors, up to a wave's 64, and a head's page of 1, 2, 4 or 8 waves of
-// them -- every page, code and key-scale address aligned to its vector; else 0.
-int quant_blocks_vectors(const barq_kv_pool* p, const barq_kv_cold* c) {
+// A compress takes head rows of a power of two of 16-byte vectors, up to a wave's 64, in pages of a power
+// of two of tokens, every page, code and key-scale address aligned to its vector: a head's page of 1, 2,
+// 4 or 8 waves' vectors as a unit, less than one wave's packed, 16 to 64 waves' split (K by columns, so
+// a row has as many vectors as the head has units).
+QuantUnits quant_units(const barq_kv_pool* p, const barq_kv_cold* c) {
+  QuantUnits q;
   const int64_t ve = 16 / p->elem_bytes;
   const uint64_t bits = (uint64_t)(uintptr_t)p->key_pages | (uint64_t)(uintptr_t)p->value_pages;
   const uint64_t cbits = (uint64_t)(uintptr_t)c->key_codes | (uint64_t)(uintptr_t)c->value_codes |
                          (uint64_t)(uintptr_t)c->key_scales;
-  if (p->head_dim % ve || (bits & 15) || (cbits & (uint64_t)(ve - 1))) return 0;
-  const int64_t vd = p->head_dim / ve;
-  if (vd > kWave || (vd & (vd - 1)) || (p->page_size * vd) % kWave) return 0;
-  const int64_t nv = p->page_size * vd / kWave;
-  return nv == 1 || nv == 2 || nv == 4 || nv == 8 ? (int)nv : 0;
+  if (p->head_dim % ve || (bits & 15) || (cbits & (uint64_t)(ve - 1))) return q;
+  const int64_t vd = p->head_dim / ve, n = p->page_size * vd;
+  if (vd > kWave || (vd & (vd - 1)) || (n & (n - 1)) || n > kWave * kWave || n > 8 * kWave * vd) return q;
+  q.nv = (int)std::min<int64_t>(std::max<int64_t>(n / kWave, 1), 8);
+  q.mode = n < kWave ? kPackedUnit : n > 8 * kWave ? kSplitUnit : kWholeUnit;
+  if (q.mode == kPackedUnit) q.log2 = __builtin_ctzll((unsigned long long)n);
+  if (q.mode == kSplitUnit) q.log2 = __builtin_ctzll((unsigned long long)(n / (8 * kWave)));
+  return q;
+}
+
+// The vectors per lane where an append quantises from its input too: whole units only.
+int quant_blocks_vectors(const barq_kv_pool* p, const barq_kv_cold* c) {
+  const QuantUnits q = quant_units(p, c);
+  return q.mode == kWholeUnit ? q.nv : 0;
 }
 
 // Quantises blocks of `batch` rows: behind an append of `tokens`, already committed, or for the rows'
-// lengths `ahead` tokens on, in order or spread.
-int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, int nv, int64_t batch, int64_t tokens,
+// lengths `ahead` tokens on, in order or (whole units) spread.
+int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, const QuantUnits& q, int64_t batch, int64_t tokens,
                         int64_t ahead, bool spread, const void* ks, const void* vs, int64_t sb, int64_t sh,
                         int64_t st, hipStream_t stream) {
   QuantArgs a;
@@ -1917,18 +1975,20 @@ int launch_quant_blocks(const barq_kv_pool* pool, const barq_kv_cold* cold, int 
   a.nnew = (int32_t)nnew;
   const int64_t vd = pool->head_dim * pool->elem_bytes / 16;
   a.vd_log2 = __builtin_ctzll((unsigned long long)vd);
+  a.mode_log2 = q.log2;
   a.div_page = FastDiv::make((uint32_t)P);
   a.div_tiles = FastDiv::make((uint32_t)(nnew + kOldTiles));
-  const bool tiled = tokens > 0 || spread;
+  const bool tiled = tokens > 0 || (spread && q.mode == kWholeUnit);
   const int64_t tiles = tiled ? batch * (nnew + kOldTiles) : batch;
   if (tiles > kI32Max) return BARQ_KV_ERR_INVALID;
   const auto fn_of = [&](auto kind) {
-    return tiled ? quant_blocks_fn_t<decltype(kind)::value>(nv) : compress_blocks_fn_t<decltype(kind)::value>(nv);
+    return tiled ? quant_blocks_fn_t<decltype(kind)::value>(q.nv) : compress_blocks_fn_t<decltype(kind)::value>(q);
   };
   const void* fn = cold->element_type == BARQ_KV_BF16   ? fn_of(std::integral_constant<int, BARQ_KV_BF16>{})
                    : cold->element_type == BARQ_KV_FP16 ? fn_of(std::integral_constant<int, BARQ_KV_FP16>{})
                                                         : fn_of(std::integral_constant<int, BARQ_KV_FP32>{});
-  const int threads = kWave * (int)std::min<int64_t>(16, 2 * pool->kv_heads);
+  const int64_t H = pool->kv_heads, packed = q.mode == kPackedUnit ? kWave >> q.log2 : 1;
+  const int threads = kWave * (int)std::min<int64_t>(16, 2 * (q.mode == kSplitUnit ? H << q.log2 : (H + packed - 1) / packed));
   void* args[] = {&a};
   return hipLaunchKernel(fn, dim3((uint32_t)tiles), dim3((uint32_t)threads), args, 0, stream) == hipSuccess
              ? BARQ_KV_OK
@@ -1993,8 +2053,8 @@ int compress_launch(const barq_kv_pool* pool, const barq_kv_cold* cold, int64_t 
                     void* stream) {
   if (!cold_ok(pool, cold) || batch < 0 || batch > pool->max_batch) return BARQ_KV_ERR_INVALID;
   if (batch == 0) return BARQ_KV_OK;
-  if (const int nv = quant_blocks_vectors(pool, cold))
-    return launch_quant_blocks(pool, cold, nv, batch, 0, ahead, spread, nullptr, nullptr, 0, 0, 0, (hipStream_t)stream);
+  if (const QuantUnits q = quant_units(pool, cold); q.nv)
+    return launch_quant_blocks(pool, cold, q, batch, 0, ahead, spread, nullptr, nullptr, 0, 0, 0, (hipStream_t)stream);
   CompressArgs a;
   a.p = *pool;
   a.c = cold_ptrs(cold);
@@ -2063,7 +2123,7 @@ int append_direct(const barq_kv_pool* pool, const barq_kv_cold* cold, const void
   if (hipLaunchKernel((const void*)&append_plan_kernel, dim3(1), dim3(kPlanThreads), args, 0,
                       (hipStream_t)stream) != hipSuccess)
     return BARQ_KV_ERR_LAUNCH;
-  return launch_quant_blocks(pool, cold, nv, batch, tokens, 0, true, key_states, value_states, stride_b, stride_h, stride_t,
+  return launch_quant_blocks(pool, cold, QuantUnits{nv}, batch, tokens, 0, true, key_states, value_states, stride_b, stride_h, stride_t,
                              (hipStream_t)stream);
 }
 
@@ -2285,6 +2345,7 @@ int append_fresh_cold(const barq_kv_pool* pool, const barq_kv_cold* cold, const 
   a.ahead = 0;
   a.nnew = (int32_t)nblk;
   a.vd_log2 = __builtin_ctzll((unsigned long long)(pool->head_dim * eb / 16));
+  a.mode_log2 = 0;
   a.div_page = FastDiv::make((uint32_t)P);
   a.div_tiles = FastDiv::make((uint32_t)nblk);
   f.out[0] = (char*)key_out;
