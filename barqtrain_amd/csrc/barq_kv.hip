@@ -61,9 +61,12 @@ constexpr int64_t kLargeLaunchTiles = 1536;
 // Stream-kernel tiles (five-wave workgroups) resident on one CU at once.
 constexpr int64_t kResidentTilesPerCU = 4;
 
-// Rows kernel: tiles resident on one CU (32 waves), and a tile's own cost in slots.
+// Rows kernel: tiles resident on one CU (32 waves), a tile's own cost in slots, and the tiles a CU up to
+// which (and past kKnownBackToBackTiles) a wave keeps one store in flight: 31 MB at 3.75 a CU 15.9 back to
+// back, 14.8 us paced; 25 MB at 4.8 13.8 and 16.4; 49 MB at 6 23.9 and 25.1, 336 MB 112 and 115.
 constexpr int64_t kRowsResidentTilesPerCU = 6;
 constexpr int64_t kRowsTileSlots = 2;
+constexpr int64_t kRowsPacedTilesPerCU = 4;
 
 template <int VB>
 struct VecT;
@@ -237,7 +240,8 @@ struct StreamArgs {
   FastDiv div_page;  // by page_size
   FastDiv div_chunks;
   FastDiv div_pieces;  // by tail pieces per (row, K or V)
-  int32_t slots;       // rows kernel: wave loads per copy wave
+  int32_t slots;       // rows kernel: wave loads per copy wave ...
+  int32_t paced;       // ... and whether a wave keeps one store in flight
   FastDiv div_loads;   // rows kernel: by wave loads per page
 };
 
@@ -943,12 +947,15 @@ __global__ void __launch_bounds__(kStreamThreads) lean_known_kernel(const Stream
 // copy wave takes `slots` consecutive slots of a (row, K or V) stream, all its loads in flight
 // before its first store; the host picks the count that gives every CU work -- a row of 256 bytes
 // cut into 64 KiB tiles filled fewer than the 256 CUs (24 rows of 1024 positions, 25 MB: 240 tiles,
-// 10.6 us; 768 of these, 7.9 us, ~4 us of it the launch and its two round trips).  Metadata and commit as in the lean kernels: from the arguments (KNOWN),
-// or read by every copy wave before the tile arrives.
+// 10.6 us; 768 of these, 7.0 us, ~4 us of it the launch and its two round trips).  Metadata and commit
+// as in the lean kernels: from the arguments (KNOWN), or read by every copy wave before the tile
+// arrives.
 //
-// A wave whose slots all hold old positions, or all new tokens, moves them without a branch or a
-// per-lane decision; the others (a row's end, padding, an unmapped page) decide per vector.  COL:
-// hv divides 64, a lane's column is the same in every slot.
+// A wave whose slots all hold old positions, or all new tokens, moves them without a per-lane
+// decision; the others (a row's end, padding, an unmapped page) choose each vector's address, loading
+// every slot at once all the same: the launch ends with its rows' ends, and loads under a condition
+// made those one round trip a slot (update of 1 x 8192 positions of 5 x 128: 12.6 -> 10.1 us; 64 x 300
+// of 5 x 64 13.6 -> 10.6).  COL: hv divides 64, a lane's column is the same in every slot.
 // ---------------------------------------------------------------------------------------------
 template <int NU, bool KNOWN, bool COL>
 __device__ __forceinline__ void lean_rows_body(const StreamArgs& a, const KnownState* ks) {
@@ -1076,27 +1083,35 @@ __device__ __forceinline__ void lean_rows_body(const StreamArgs& a, const KnownS
       val[u] = ld_stream<V>(in_row + ((int64_t)(s - len) * ist + ih));
     }
   } else {
+    // Every lane loads -- a new token's vector, else the page's (page 0's where there is none), replaced
+    // below by zeros where nothing was written: a load under a condition waits before the next slot's.
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
-      val[u] = zero_vec<V>();
-      if (u < n) {
-        const int pk = slot_page(u), part = slot_part(u, pk);
-        int tok;
-        uint32_t oh, ih;
-        lane_at(part, tok, oh, ih);
-        const int s = (pg0 + pk) * P + tok;
-        const int pg = __builtin_amdgcn_readlane(page, pk);
-        if (s < S) {
-          if ((unsigned)(s - len) < (unsigned)T) {
-            val[u] = ld_stream<V>(in_row + ((int64_t)(s - len) * ist + ih));
-          } else if (s < hw && pg >= 0) {
-            val[u] = ld_stream<V>(pages + (int64_t)pg * a.page_bytes + (uint32_t)((part * kWave + lane) * 16));
-          }
-        }
-      }
+      const int i = min(u, n - 1);
+      const int pk = slot_page(i), part = slot_part(i, pk);
+      int tok;
+      uint32_t oh, ih;
+      lane_at(part, tok, oh, ih);
+      const int s = (pg0 + pk) * P + tok;
+      const int pg = __builtin_amdgcn_readlane(page, pk);
+      const char* at = pages + (int64_t)max(pg, 0) * a.page_bytes + (uint32_t)((part * kWave + lane) * 16);
+      if ((unsigned)(s - len) < (unsigned)T && s < S) at = in_row + ((int64_t)(s - len) * ist + ih);
+      val[u] = ld_stream<V>(at);
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int i = min(u, n - 1);
+      const int pk = slot_page(i), part = slot_part(i, pk);
+      int tok;
+      uint32_t oh, ih;
+      lane_at(part, tok, oh, ih);
+      const int s = (pg0 + pk) * P + tok;
+      const bool written = (unsigned)(s - len) < (unsigned)T || (s < hw && __builtin_amdgcn_readlane(page, pk) >= 0);
+      if (!written) val[u] = zero_vec<V>();
     }
   }
-  const bool paced = gridDim.x > kKnownBackToBackTiles;
+  // (a tile of both kinds is a row's end, which the launch waits for: its stores go back to back)
+  const bool paced = a.paced && (all_old || all_new);
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     if (u < n) {
@@ -2256,6 +2271,10 @@ int run_stream(const barq_kv_pool* pool, const void* ks, const void* vs, int64_t
   // least work on those -- tiles times slots, a tile's own cost (metadata, its first round trip)
   // counted as kRowsTileSlots more -- while the tiles are resident at once, else 8.  (24 rows of
   // 1024 x 256 B, K and V: 2 / 3 / 4 / 8 slots, 6 / 4.1 / 3 / 1.5 tiles a CU, 9.6 / 8.7 / 8.0 / 8.5 us.)
+  // The any-geometry kernel -> this one, updates of one token, us: 16 vectors a row 9.7 -> 6.4 at 24 x
+  // 1021, 27 -> 26 at 8 x 16384; 80 11.4 -> 9.6 at 1 x 8192, 147 -> 115 at 64 x 2048, 11.6 -> 12.0 at 16 x
+  // 650 (whose 448 large tiles happen to fill the CUs); 192 55 -> 53 at 24 x 1021; 512 58 -> 48 at 1 x
+  // 8192, 156 -> 133 at 24 x 1021.
   int64_t row_slots = 0, row_chunks = 0;
   const auto block32 = [&](int64_t stride, int64_t head_span) {
     return stride >= 0 && stride <= kI32Max && P * stride + head_span <= kI32Max;
@@ -2352,10 +2371,11 @@ int run_stream(const barq_kv_pool* pool, const void* ks, const void* vs, int64_t
   const bool rounds = fast && ncu > 0 && grid > kResidentTilesPerCU * ncu;
   int rc;
   if (row_slots > 0) {
+    const int64_t row_grid = 2 * batch * row_chunks;
     a.slots = (int32_t)row_slots;
+    a.paced = row_grid > kKnownBackToBackTiles && row_grid <= kRowsPacedTilesPerCU * ncu;
     a.div_loads = FastDiv::make((uint32_t)(P * hv / kWave));
     a.div_chunks = FastDiv::make((uint32_t)row_chunks);
-    const int64_t row_grid = 2 * batch * row_chunks;
     a.nsub = (int32_t)std::min<int64_t>(row_grid, BARQ_KV_CTRL_SUBCOUNTERS);
     const KnownState* k = known && tokens > 0 && a.commit_in_kernel && !a.seq_from_device ? known : nullptr;
     rc = launch_rows_kernel(row_slots <= 2 ? 2 : row_slots <= 4 ? 4 : 8, kWave % hv == 0, dim3((uint32_t)row_grid), &a,
