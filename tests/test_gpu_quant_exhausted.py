@@ -16,17 +16,18 @@ NAMES = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "f32"}
 DIRECT = 8
 
 
-# blocks of a wave's vectors and of less, a row of more blocks than one pass looks at, one row's workgroup each
+# blocks of a wave's vectors and of less; rows of more blocks than one pass looks at, than two, than 64
 @pytest.mark.parametrize("B,H,D,P,blocks,num_cold,dtype",
                          [(3, 8, 128, 16, 6, 7, torch.bfloat16), (3, 2, 64, 16, 6, 1, torch.float16),
                           (4, 3, 256, 16, 5, 10, torch.bfloat16), (3, 4, 64, 16, 6, 11, torch.float32),
                           (2, 2, 64, 16, 300, 400, torch.bfloat16), (1, 2, 64, 16, 300, 270, torch.float16),
+                          (2, 2, 64, 16, 900, 1300, torch.bfloat16), (1, 1, 64, 1, 17000, 16950, torch.bfloat16),
                           (2, 1, 8, 4, 6, 5, torch.float32)])
 def test_compress_quantises_the_leading_blocks(capi, B, H, D, P, blocks, num_cold, dtype):
     gen = torch.Generator().manual_seed(num_cold)
     pool = CColdPool(window=0, num_cold=num_cold, max_batch=B, max_blocks=blocks, page_size=P, heads=H, dim=D, dtype=dtype)
     oracle = q.QuantLayerOracle(B, blocks * P, P, 0, NAMES[dtype])
-    n = (blocks - 1) * P + 3
+    n = (blocks - 1) * P + min(3, P)
     k, v = hf_layout(B, H, n, D, dtype, gen), hf_layout(B, H, n, D, dtype, gen)
     for calls in range(2):  # the second finds the store empty
         if calls == 0:
@@ -43,7 +44,7 @@ def test_compress_quantises_the_leading_blocks(capi, B, H, D, P, blocks, num_col
     mine = np.repeat(cold, P, axis=1)[:, None, :n, None]
     for g, e, w in zip(got, exact, read):
         assert np.array_equal(to_bits(g), np.where(mine, w, e))
-    if dtype != torch.float32 and D != 256:
+    if dtype != torch.float32 and D != 256 and P % 16 == 0:
         query = hf_layout(B, 2 * H, 1, D, dtype, gen)
         out = attend_cold(pool, query.cuda())
         want = decode_attention_reference(*(x.double().cpu().numpy() for x in (query, *got)), [n] * B, D ** -0.5)
