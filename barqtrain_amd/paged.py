@@ -268,22 +268,25 @@ class PagePool:
         returns (key_out, value_out, pages taken), or pages taken < 0 when the call must take the
         checked path (which raises the exact error, or handles an empty call), and the longest row
         after the call."""
-        backend = _gpu_backend()
+        handle = self._packed()
         limit = self.capacity if max_length is None else int(max_length)
-        ko, vo, need, worst = backend.pool_step_(self._packed(backend)[1], self.key_pages, key_states, value_states,
-                                                 self.lens, self.hw, self.free_count, self.free_exact, limit, flags,
-                                                 gather)
+        ko, vo, need, worst = handle[3].pool_step_(handle[1], self.key_pages, key_states, value_states, self.lens, self.hw,
+                                                   self.free_count, self.free_exact, limit, flags, gather)
         if need >= 0:
             self.free_count -= need
         return ko, vo, need, worst
 
-    def _packed(self, backend):
-        """(generation, pool, cold store or None): the pool's tensors packed for the binding's step
-        calls, packed again when they are replaced."""
+    def _packed(self):
+        """(generation, pool, cold store or None, the binding): the pool's tensors packed for the
+        binding's step calls, packed again when they are replaced."""
         handle = self._handle
         if handle is None or handle[0] != self.generation:
-            handle = self._handle = (self.generation, backend.pool_group([self.tensors]), None)
+            backend = _gpu_backend()
+            handle = self._handle = (self.generation, backend.pool_group([self.tensors]), self._packed_cold(backend), backend)
         return handle
+
+    def _packed_cold(self, backend):
+        return None
 
     def step(self, key_states: torch.Tensor, value_states: torch.Tensor, max_length: int, gather: bool):
         """An eager decode step: ``(K, V, longest row)`` of an update (K and V None for an append),
@@ -336,7 +339,7 @@ class PagePool:
         t = self.tensors
         ops = self._ops()
         if not (self.on_gpu and self.free_exact and ops.pool_append_rows_(
-                self._packed(ops)[1], self.key_pages, k, v, rows, self.lens, self.hw, self.free_count)):
+                self._packed()[1], self.key_pages, k, v, rows, self.lens, self.hw, self.free_count)):
             for i, row in enumerate(rows):
                 one = t[:2] + [t[2][row:row + 1], t[3][row:row + 1], t[4][row:row + 1]] + t[5:]
                 ops.pool_append_(one, k[i:i + 1], v[i:i + 1])
@@ -557,10 +560,9 @@ class PagePool:
         or None when `attend` has to look at the call (or to allocate the workspace)."""
         if self.device.type != "cuda" or self._attn_ws is None:
             return None
-        backend = _gpu_backend()
         scale = 1.0 / math.sqrt(self.head_dim) if scale is None else float(scale)
-        handle = self._packed(backend)
-        return backend.pool_attend(handle[1], handle[2], self.key_pages, query, self.lens, scale, self._attn_ws)
+        handle = self._packed()
+        return handle[3].pool_attend(handle[1], handle[2], self.key_pages, query, self.lens, scale, self._attn_ws)
 
     def _attention_call(self, backend, query, out, scale, max_seq, split_tokens, ws):
         backend.pool_decode_attention(self.tensors, query, out, scale, max_seq, split_tokens, ws)
@@ -694,18 +696,13 @@ class QuantPagePool(PagePool):
         self.cold_free -= moved
         self.free_count += moved  # each quantised block returned its full-precision page
 
-    def _packed(self, backend):
-        handle = self._handle
-        if handle is None or handle[0] != self.generation:
-            handle = self._handle = (self.generation, backend.pool_group([self.tensors]),
-                                     backend.cold_group(self.tensors, self.cold_tensors, self.window))
-        return handle
+    def _packed_cold(self, backend):
+        return backend.cold_group(self.tensors, self.cold_tensors, self.window)
 
     def _step(self, key_states, value_states, max_length, flags, gather):
-        backend = _gpu_backend()
-        handle = self._packed(backend)
+        handle = self._packed()
         limit = self.capacity if max_length is None else int(max_length)
-        ko, vo, need, worst, moved = backend.pool_step_cold_(
+        ko, vo, need, worst, moved = handle[3].pool_step_cold_(
             handle[1], handle[2], self.key_pages, key_states, value_states, self.lens, self.hw, self.cold_blocks,
             self.free_count, self.free_exact, self.cold_free, self.chunk, limit, flags, gather)
         if need >= 0:
@@ -1201,10 +1198,9 @@ def reset_layers(pools: Sequence[PagePool]) -> None:
         for p in pools:
             p.reset()
         return
-    backend = _gpu_backend()
-    packed = [p._packed(backend) for p in pools]
+    packed = [p._packed() for p in pools]
     colds = [h[2] for h in packed] if getattr(pools[0], "quantized", False) else []
-    backend.reset_layers_([h[1] for h in packed], colds, pools[0].key_pages)
+    packed[0][3].reset_layers_([h[1] for h in packed], colds, pools[0].key_pages)
     for p in pools:
         p._emptied()
 
