@@ -327,8 +327,8 @@ __global__ void __launch_bounds__(kThreads) compress_kernel(const CompressArgs a
 // tops, which no other part of the launch moves the other way.
 //
 // Bound: HBM (the input read once, codes and scales written once), then the round trips of a
-// workgroup's only block.  A 16 x 1000-token prompt of the 8 x 128 bf16 shape: 24.1 us for 95 MB
-// after a 6.8 us plan, against 16 chunks of an append and a compress each, 9.2 + 33 us.
+// workgroup's only block.  A 16 x 1000-token prompt of the 8 x 128 bf16 shape: 25.6 us for 95 MB
+// after a 7.1 us plan, against 16 chunks of an append and a compress each, 9.2 + 33 us.
 // ---------------------------------------------------------------------------------------------
 
 // Tiles per row that look for older hot blocks: an append of 64 tokens pushes four out of the window
@@ -1229,8 +1229,8 @@ __device__ __forceinline__ typename Vec<KIND, 8>::Out exact8(uint32_t w0, uint32
 // few of a block's units, the block's first also writing its table entry (and row 0's the tops).
 //
 // Bound: HBM (input read once, codes and output written once).  A 16 x 1000-token prompt of the 8 x 128
-// bf16 shape: 30.7 us for 163 MB (5.3 TB/s) against 6.8 (plan) + 24.1 + 17.7 (gather, codes from cache);
-// without output 21.5 against 30.9.
+// bf16 shape: 31 us for 163 MB (5.3 TB/s) against 7.1 (plan) + 25.6 + 17.7 (gather, codes from cache);
+// without output 20.7 against 32.7.
 // ---------------------------------------------------------------------------------------------
 
 struct FreshArgs {

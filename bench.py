@@ -797,7 +797,7 @@ def quant_leg(cfg, wl, steps, dev, bf16_ms_per_step, window=128, reps=10, probe=
     full = 2 * B * mb * P * H * D * esize
     return {
         "kernels": ("update_cold_lanes_kernel (append + dequantising gather, one launch) per layer, and "
-                    "quant_blocks_kernel when blocks leave the window; graph-replayed"),
+                    "compress_blocks_kernel when blocks leave the window; graph-replayed"),
         "format": f"fp8 E4M3 codes, E8M0 scales (keys per channel, values per token over a page), "
                   f"residual window {window} tokens",
         "us_per_step_all_layers": round(ms * 1e3, 1),
